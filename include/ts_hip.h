@@ -375,16 +375,23 @@ int ts_hip_matmul(const float *a, const float *b, float *c, size_t m, size_t n, 
  *   trans_b == 0: B(k,j) = B[k*ldb + j]   (B stored [K][ldb])
  *   trans_b == 1: B(k,j) = B[j*ldb + k]   (B stored [N][ldb], i.e. B^T view)
  *   C(i,j) = C[i*ldc + j]
- * fp32 inputs, fp32 MFMA accumulation (v_mfma_f32_16x16x4_f32 when M and N
- * are multiples of 256, K of 32 and the grid has a 256x256 tile per CU; else
- * v_mfma_f32_32x32x2_f32: the two add k in different groupings, so a product's
- * last bits depend on which it takes; every entry point below takes the same
- * one for the same shape, layout and alignment).  M, N, K and
+ * fp32 inputs and accumulation.  Products of 3e9 operations and more run on
+ * the f16 matrix cores: each value, scaled into range by its row of op(A) or
+ * column of op(B), as the sum of two f16 values (within 2^-24 of itself or
+ * 2^-40 of its row's largest), three f16 products summed in fp32 -- closer to
+ * the exact product than the fp32 instructions.  Output tiles whose rows or
+ * columns hold an infinity or spread too far for that, and smaller products,
+ * run on the fp32 instructions (v_mfma_f32_16x16x4_f32 when M and N are
+ * multiples of 256, K of 32 and the grid has a 256x256 tile per CU; else
+ * v_mfma_f32_32x32x2_f32).  The kinds add k in different groupings, so a
+ * product's last bits depend on which it takes; every entry point below takes
+ * the same one for the same shape, layout and alignment.  M, N, K and
  * the leading dimensions must be below 2^31 (TS_HIP_EINVAL otherwise).  For
  * few output tiles with a long K (e.g. M = 32, K = 784) the call splits K and
  * takes a temporary of up to 16*M*N floats from the stream-ordered allocator
  * (hipMallocAsync / hipFreeAsync on `stream`); where that allocator is
- * unavailable it runs unsplit. */
+ * unavailable it runs unsplit, as does a product on the f16 matrix cores while
+ * a graph is recorded. */
 int ts_hip_gemm(int trans_a, int trans_b, size_t M, size_t N, size_t K, const float *A,
                 size_t lda, const float *B, size_t ldb, float *C, size_t ldc, void *stream);
 
@@ -392,7 +399,7 @@ int ts_hip_gemm(int trans_a, int trans_b, size_t M, size_t N, size_t K, const fl
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  Same arguments,
  * kernels and results (bit for bit) as ts_hip_gemm; a split product's
- * temporary comes from a fixed device array of 2^21 floats (8 MiB) that each
+ * temporary comes from a fixed device array of 2^23 floats (32 MiB) that each
  * device holds for the life of the process, which every split this device
  * can choose fits (a product needing more returns TS_HIP_ESCRATCH).  The
  * array is shared by all calls on a device: calls that overlap on one device
@@ -418,7 +425,8 @@ size_t ts_hip_gemm_workspace_floats(size_t M, size_t N, size_t K);
  * Bit-identical to ts_hip_gemm followed by ts_hip_bias_add, ts_hip_relu and
  * ts_hip_relu_backward(mask, C, C).  A split product (see
  * ts_hip_gemm_workspace_floats) uses `workspace` (device, at least that many
- * floats; TS_HIP_EWORKSPACE if fewer) as its temporary, so the call allocates
+ * floats; with fewer, one on the f16 matrix cores runs unsplit and the others
+ * return TS_HIP_EWORKSPACE) as its temporary, so the call allocates
  * nothing and can be recorded into a HIP graph; with workspace == NULL it
  * allocates as ts_hip_gemm does. */
 int ts_hip_gemm_fused(int trans_a, int trans_b, size_t M, size_t N, size_t K, const float *A, size_t lda,
