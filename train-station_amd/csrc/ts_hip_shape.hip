@@ -6,7 +6,12 @@
 // broadcast_gather: out[i] = src[offset of i's coordinates], with the source
 // strides of broadcast axes set to 0 -- the reference materialises the same
 // values with broadcast_copy_data.  HBM-bound: 4 B written per element, the
-// source read through the caches.
+// source read through the caches.  Neighbouring axes that are both repeated, or
+// both copied, are merged first ([8192, 1] over [8192, 1024] is two axes, a bias
+// over any batch two); below 2^31 elements a thread then writes four
+// consecutive ones (broadcast_quads) and finds their coordinates with
+// multiplications: a 64-bit division per element and axis had bound the copy
+// (8192 x 1024: 24 us, now 8).
 //
 // reduce_axes: output element o (keepdim layout) sums the input elements
 // whose kept coordinates equal o's, in f64, in a fixed order: G lanes per
@@ -37,6 +42,68 @@ __global__ __launch_bounds__(kBlock) void broadcast_gather(const float *__restri
         }
         const float v = src[off];
         out[i] = use_scale ? v * scale : v;
+    }
+}
+
+// x / d for x < 2^31: the quotient's multiplier is 2^32 (2^l - d) / d + 1 with
+// 2^l the power of two at or above d (Granlund and Montgomery, "Division by
+// invariant integers using multiplication").
+struct FastDiv {
+    uint32_t d, m, l;
+};
+static FastDiv fast_div(uint32_t d) {
+    FastDiv f{d, 0, 0};
+    while (f.l < 31 && (uint32_t(1) << f.l) < d) ++f.l;
+    f.m = static_cast<uint32_t>(((uint64_t(1) << 32) * ((uint64_t(1) << f.l) - d)) / d + 1);
+    return f;
+}
+__device__ __forceinline__ uint32_t quotient(uint32_t x, const FastDiv &f) { return (__umulhi(x, f.m) + x) >> f.l; }
+
+struct QuadLayout {
+    int rank;                    // merged axes, innermost first
+    FastDiv dim[kMaxRank];
+    uint32_t stride[kMaxRank];   // in the source; 0 repeated
+};
+
+__device__ __forceinline__ uint32_t quad_offset(const QuadLayout &L, uint32_t i) {
+    uint32_t off = 0;
+#pragma unroll
+    for (int k = 0; k < kMaxRank; ++k) {
+        if (k < L.rank - 1) {
+            const uint32_t q = quotient(i, L.dim[k]);
+            off += (i - q * L.dim[k].d) * L.stride[k];
+            i = q;
+        }
+    }
+    return off + i * L.stride[L.rank - 1];
+}
+
+// INNER: the innermost axis is a multiple of four long, so a thread's four
+// elements share the outer coordinates.  VEC: out is 16-byte aligned.
+template <bool INNER, bool VEC>
+__global__ __launch_bounds__(kBlock) void broadcast_quads(const float *__restrict__ src, float *__restrict__ out,
+                                                          uint32_t n, QuadLayout L, float scale, int use_scale) {
+    const uint32_t i = (blockIdx.x * kBlock + threadIdx.x) * 4;
+    if (i >= n) return;
+    f4v_t v;
+    if (INNER) {
+        const uint32_t off = quad_offset(L, i), s = L.stride[0];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[c] = src[off + c * s];
+    } else {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[c] = src[quad_offset(L, min(i + c, n - 1))];
+    }
+    if (use_scale) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[c] = v[c] * scale;
+    }
+    if (VEC && i + 3 < n) {
+        *reinterpret_cast<f4v_t *>(out + i) = v;
+    } else {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (i + c < n) out[i + c] = v[c];
     }
 }
 
@@ -74,8 +141,23 @@ __global__ __launch_bounds__(kBlock) void reduce_axes(const float *__restrict__ 
     const int lane = threadIdx.x % G;
     double acc = 0.0;
     if (o < R.n_out) {
-        const uint64_t base = kept_offset(R, o);
-        for (uint64_t r = lane; r < R.n_red; r += G) acc += static_cast<double>(x[base + red_offset(R, r)]);
+        const float *p = x + kept_offset(R, o);
+        if (R.red_rank == 1) {  // uniform: the reduced axes are one (merged)
+            const uint64_t step = G * R.red_stride[0];
+            p += lane * R.red_stride[0];
+            uint64_t r = lane;
+            // eight loads in flight, added in order
+            for (; r + 7 * G < R.n_red; r += 8 * G, p += 8 * step) {
+                float v[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) v[k] = p[k * step];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) acc += static_cast<double>(v[k]);
+            }
+            for (; r < R.n_red; r += G, p += step) acc += static_cast<double>(*p);
+        } else {
+            for (uint64_t r = lane; r < R.n_red; r += G) acc += static_cast<double>(p[red_offset(R, r)]);
+        }
     }
     if (G >= 64) {
 #pragma unroll
@@ -224,6 +306,38 @@ int ts_hip_broadcast_copy(const float *src, const size_t *src_dims, size_t src_r
         L.dims[0] = 1;
         L.src_stride[0] = 0;
     }
+    if (n < (size_t(1) << 31)) {
+        // merged axes, innermost first; axes of one element take no part
+        QuadLayout Q{};
+        uint64_t len[kMaxRank], str[kMaxRank];
+        for (int k = L.rank - 1; k >= 0; --k) {
+            if (L.dims[k] == 1) continue;
+            const int t = Q.rank - 1;
+            if (Q.rank && (str[t] == 0 ? L.src_stride[k] == 0 : L.src_stride[k] == str[t] * len[t])) {
+                len[t] *= L.dims[k];
+            } else {
+                len[Q.rank] = L.dims[k];
+                str[Q.rank++] = L.src_stride[k];
+            }
+        }
+        if (Q.rank == 0) {
+            len[0] = 1;
+            str[Q.rank++] = 0;
+        }
+        for (int k = 0; k < Q.rank; ++k) {
+            Q.dim[k] = fast_div(static_cast<uint32_t>(len[k]));
+            Q.stride[k] = static_cast<uint32_t>(str[k]);
+        }
+        const bool inner = len[0] % 4 == 0, vec = aligned16(out);
+        const dim3 grid(static_cast<unsigned>((n + 4 * kBlock - 1) / (4 * kBlock))), block(kBlock);
+        hipStream_t s = as_stream(stream);
+        const uint32_t n32 = static_cast<uint32_t>(n);
+        if (inner && vec) launch((broadcast_quads<true, true>), grid, block, 0, s, src, out, n32, Q, scale, use_scale);
+        else if (inner) launch((broadcast_quads<true, false>), grid, block, 0, s, src, out, n32, Q, scale, use_scale);
+        else if (vec) launch((broadcast_quads<false, true>), grid, block, 0, s, src, out, n32, Q, scale, use_scale);
+        else launch((broadcast_quads<false, false>), grid, block, 0, s, src, out, n32, Q, scale, use_scale);
+        return launch_status();
+    }
     launch(broadcast_gather, dim3(grid_for(n)), dim3(kBlock), 0, as_stream(stream), src, out, n, L,
                        scale, use_scale);
     return launch_status();
@@ -243,16 +357,25 @@ int ts_hip_reduce_sum(const float *x, const size_t *dims, size_t rank, unsigned 
     n_in = stride;
     R.n_out = 1;
     R.n_red = 1;
-    for (size_t k = 0; k < rank; ++k) {
-        if ((reduce_mask >> k) & 1u) {
-            R.red_dims[R.red_rank] = dims[k];
-            R.red_stride[R.red_rank++] = st[k];
-            R.n_red *= dims[k];
+    // neighbouring axes of a kind merged (the same element order), axes of one
+    // element left out
+    auto axis = [](int &r, uint64_t *d, uint64_t *s, uint64_t len, uint64_t stride, bool joins) {
+        if (joins) {
+            d[r - 1] *= len;
+            s[r - 1] = stride;
         } else {
-            R.kept_dims[R.kept_rank] = dims[k];
-            R.kept_stride[R.kept_rank++] = st[k];
-            R.n_out *= dims[k];
+            d[r] = len;
+            s[r++] = stride;
         }
+    };
+    int last = -1;  // the kind of the last axis taken
+    for (size_t k = 0; k < rank; ++k) {
+        const int kind = (reduce_mask >> k) & 1u;
+        (kind ? R.n_red : R.n_out) *= dims[k];
+        if (dims[k] == 1) continue;
+        if (kind) axis(R.red_rank, R.red_dims, R.red_stride, dims[k], st[k], last == 1);
+        else axis(R.kept_rank, R.kept_dims, R.kept_stride, dims[k], st[k], last == 0);
+        last = kind;
     }
     if (R.n_out == 0) return TS_HIP_OK;
     if (!out) return TS_HIP_EINVAL;
