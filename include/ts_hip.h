@@ -375,8 +375,9 @@ int ts_hip_matmul(const float *a, const float *b, float *c, size_t m, size_t n, 
  *   trans_b == 0: B(k,j) = B[k*ldb + j]   (B stored [K][ldb])
  *   trans_b == 1: B(k,j) = B[j*ldb + k]   (B stored [N][ldb], i.e. B^T view)
  *   C(i,j) = C[i*ldc + j]
- * fp32 inputs and accumulation.  Products of 3e9 operations and more run on
- * the f16 matrix cores: each value, scaled into range by its row of op(A) or
+ * fp32 inputs and accumulation.  Products of 2.2e9 operations and more (1.5e9
+ * where M, N or K is no multiple of 4; not the untransposed ones that the
+ * 16x16x4 kernel below takes) run on the f16 matrix cores: each value, scaled into range by its row of op(A) or
  * column of op(B), as the sum of two f16 values (within 2^-24 of itself or
  * 2^-40 of its row's largest), three f16 products summed in fp32 -- closer to
  * the exact product than the fp32 instructions.  Output tiles whose rows or
@@ -399,7 +400,7 @@ int ts_hip_gemm(int trans_a, int trans_b, size_t M, size_t N, size_t K, const fl
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  Same arguments,
  * kernels and results (bit for bit) as ts_hip_gemm; a split product's
- * temporary comes from a fixed device array of 2^23 floats (32 MiB) that each
+ * temporary comes from a fixed device array of 9 * 2^20 floats (36 MiB) that each
  * device holds for the life of the process, which every split this device
  * can choose fits (a product needing more returns TS_HIP_ESCRATCH).  The
  * array is shared by all calls on a device: calls that overlap on one device
@@ -407,9 +408,10 @@ int ts_hip_gemm(int trans_a, int trans_b, size_t M, size_t N, size_t K, const fl
 int ts_hip_gemm_noalloc(int trans_a, int trans_b, size_t M, size_t N, size_t K, const float *A,
                         size_t lda, const float *B, size_t ldb, float *C, size_t ldc, void *stream);
 
-/* Floats of workspace a split product needs (the temporary ts_hip_gemm takes
- * from the stream-ordered allocator for few output tiles with a long K):
- * 0 when the product M x N x K is not split. */
+/* Floats of workspace a product can use: the temporary of a K split over
+ * workgroups (what ts_hip_gemm takes from the stream-ordered allocator), and on
+ * the f16 matrix cores a scan of the operands, without which its workgroups
+ * scan (the same result, slower).  0 when the product M x N x K uses none. */
 size_t ts_hip_gemm_workspace_floats(size_t M, size_t N, size_t K);
 
 /* The same product with the elementwise ops that follow it fused into the
@@ -425,7 +427,7 @@ size_t ts_hip_gemm_workspace_floats(size_t M, size_t N, size_t K);
  * Bit-identical to ts_hip_gemm followed by ts_hip_bias_add, ts_hip_relu and
  * ts_hip_relu_backward(mask, C, C).  A split product (see
  * ts_hip_gemm_workspace_floats) uses `workspace` (device, at least that many
- * floats; with fewer, one on the f16 matrix cores runs unsplit and the others
+ * floats; with fewer, one on the f16 matrix cores does without and the others
  * return TS_HIP_EWORKSPACE) as its temporary, so the call allocates
  * nothing and can be recorded into a HIP graph; with workspace == NULL it
  * allocates as ts_hip_gemm does. */

@@ -1631,8 +1631,15 @@ struct GemmPlan {
         if (f16.slices < 2) return;
         f16.slices = 1;
         f16.kslice = 0;
-        f16.partial_floats = split_floats = 0;
+        f16.partial_floats = 0;
+        drop_scan();
     }
+    // Without a scan of its own (that launch needs a workspace from the caller).
+    void drop_scan() {
+        f16.scan_floats = 0;
+        if (f16.on) split_floats = f16.partial_floats;
+    }
+    size_t scan_offset() const { return (f16.partial_floats + 3) & ~size_t(3); }
     size_t part_offset() const { return (split_floats + 1) & ~size_t(1); }
     size_t total() const { return part_floats ? part_offset() + part_floats : split_floats; }
 };
@@ -1668,7 +1675,7 @@ static GemmPlan gemm_plan(int trans_a, int trans_b, size_t M, size_t N, size_t K
         // their 128 x 128 tiles append the fp32 tiles' column strips; past
         // those a column-sum pass follows
         p.cs_kernel = colsum && trans_a && !trans_b && p.f16.tile == 128;
-        p.split_floats = p.f16.partial_floats;
+        p.split_floats = p.f16.scan_floats ? p.scan_offset() + p.f16.scan_floats : p.f16.partial_floats;
         p.part_floats = colsum && !p.cs_kernel ? 2 * colsum_chunk_count(K) * N : 0;
     }
     return p;
@@ -1767,9 +1774,11 @@ static int gemm_plain(int trans_a, int trans_b, size_t M, size_t N, size_t K, co
     if (!A || !B || lda < (trans_a ? M : K) || ldb < (trans_b ? K : N)) return TS_HIP_EINVAL;
     GemmPlan plan = gemm_plan(trans_a, trans_b, M, N, K, colsum != nullptr, split_lds_ok(lda, ldb, ldc));
     hipStream_t st = as_stream(stream);
-    // without room for its slices (a caller's workspace that is smaller, or
-    // none while a graph is recorded) a product on the f16 matrix cores runs
-    // whole
+    // A product on the f16 matrix cores without room for its scan (no workspace
+    // of the caller's, or a smaller one) scans in its workgroups, and without
+    // room for its slices (a smaller one yet, or none while a graph is
+    // recorded) runs whole.
+    if (plan.f16.on && (!ws || ws_floats < plan.total() || (reinterpret_cast<uintptr_t>(ws) & 15))) plan.drop_scan();
     if (plan.f16.slices > 1 && (ws ? ws_floats < plan.total() : capturing(st))) plan.unslice();
     const size_t need = plan.total();
     float *W = ws;
@@ -1821,7 +1830,7 @@ static int gemm_plain(int trans_a, int trans_b, size_t M, size_t N, size_t K, co
         if (xb) g.xb = *xb;
         gemm_operands(g, M, N, K, A, lda, B, ldb, C, ldc);
         if (plan.cs_kernel) g.colsum = colsum;
-        status = launch_split(plan.f16, trans_a, trans_b, g, 1, W, st);
+        status = launch_split(plan.f16, trans_a, trans_b, g, 1, W, plan.f16.scan_floats ? W + plan.scan_offset() : nullptr, st);
         if (status == TS_HIP_OK && colsum && !plan.cs_kernel)
             status = launch_colsum(B, nullptr, K, N, ldb, colsum, reinterpret_cast<float *>(part), plan.part_floats,
                                    stream);
@@ -1881,8 +1890,9 @@ extern "C" int ts_hip_gemm(int trans_a, int trans_b, size_t M, size_t N, size_t 
 // ---- allocation-free form --------------------------------------------------
 //
 // ts_hip_gemm_noalloc takes a product's workspace from this fixed device
-// array instead of the stream-ordered allocator.  A K split on the f16 matrix
-// cores asks for at most 2^23 floats (32 MiB; split_plan chooses no other).  An MFMA split runs only
+// array instead of the stream-ordered allocator.  A product on the f16 matrix
+// cores asks for at most 2^23 floats of partial products and 2^20 of its scan
+// (36 MiB; split_plan chooses no other).  An MFMA split runs only
 // while 4 * (64x64 tiles) < CUs with slices * tiles <= 2 * CUs, so it never
 // needs more than 2 * CUs * 64 * 64 floats: 2^21 (8 MiB) on the 256 CUs of an
 // MI355X; a skinny split (N <= 16) has fewer 64-row groups than CUs and at
@@ -1890,7 +1900,7 @@ extern "C" int ts_hip_gemm(int trans_a, int trans_b, size_t M, size_t N, size_t 
 // of the process.  Calls that overlap on one device (several streams) share
 // it and race; the split slices are fully written before they are read, so
 // nothing needs clearing between calls.
-static constexpr size_t kScratchFloats = size_t(1) << 23;
+static constexpr size_t kScratchFloats = 9 * (size_t(1) << 20) + 64;
 static __device__ __align__(256) float scratch[kScratchFloats];
 
 namespace tship {
@@ -1933,7 +1943,10 @@ extern "C" int ts_hip_gemm_noalloc(int trans_a, int trans_b, size_t M, size_t N,
 }
 
 extern "C" size_t ts_hip_gemm_workspace_floats(size_t M, size_t N, size_t K) {
-    return gemm_plan(0, 0, M, N, K, false).total();
+    // the layout that takes most: NT products run on the f16 matrix cores where
+    // NN ones of an exact tiling do not
+    const size_t nn = gemm_plan(0, 0, M, N, K, false).total(), nt = gemm_plan(0, 1, M, N, K, false).total();
+    return nn > nt ? nn : nt;
 }
 
 extern "C" int ts_hip_gemm_fused(int trans_a, int trans_b, size_t M, size_t N, size_t K, const float *A,
@@ -2086,7 +2099,8 @@ extern "C" int ts_hip_gemm_batched(int trans_a, int trans_b, size_t M, size_t N,
     const SplitPlan plan = split_plan(M, N, K, batches);
     if (plan.on && A && B && lda >= (trans_a ? M : K) && ldb >= (trans_b ? K : N) && split_lds_ok(lda, ldb, ldc)) {
         gemm_operands(g, M, N, K, A, lda, B, ldb, C, ldc);
-        return launch_split(plan, trans_a, trans_b, g, static_cast<unsigned>(batches), nullptr, as_stream(stream));
+        return launch_split(plan, trans_a, trans_b, g, static_cast<unsigned>(batches), nullptr, nullptr,
+                            as_stream(stream));
     }
     return gemm_launch(trans_a, trans_b, M, N, K, A, lda, B, ldb, C, ldc, g, batches, stream);
 }

@@ -497,16 +497,20 @@ constexpr int prefetch_tiles() { return BM >= 256 ? 1 : 4; }
 
 // What such a product takes: 256 x 256 or 128 x 128 tiles, and K in `slices` of
 // kslice (0: whole), whose partial products need partial_floats of workspace.
+// With scan_floats more the operands are scanned by a launch of their own, the
+// faster (the same result without).
 struct SplitPlan {
     bool on = false;
     int tile = 0;
     int slices = 1;
     int kslice = 0;
-    size_t partial_floats = 0;
+    size_t partial_floats = 0, scan_floats = 0;
 };
 SplitPlan split_plan(size_t M, size_t N, size_t K, size_t batches);
 // The product (a split one by its slices' partial products in `partial`); g as for the
 // fp32 kernels (its colsum is written for 128 x 128 tiles, not for 256 x 256).
-int launch_split(const SplitPlan &plan, int ta, int tb, GemmArgs g, unsigned batches, float *partial, hipStream_t s);
+// scan: scan_floats of workspace (16-byte aligned), or null.
+int launch_split(const SplitPlan &plan, int ta, int tb, GemmArgs g, unsigned batches, float *partial, float *scan,
+                 hipStream_t s);
 
 }  // namespace tship

@@ -17,14 +17,13 @@
 // element's error is then at most 2^-24 of itself or 2^-40 of its row's
 // largest, whichever is larger.  A workgroup first scans its rows and columns
 // over its k for the largest magnitude and the mean exponent of the non-zero
-// elements (a fifth to a quarter of the kernel's time; it reads what the product
-// will, from L2.  A scan of its own before the product would read each operand
-// once and cost 6% of the largest products, but a second launch and a workspace
-// for every one).  A tile with a row or column that holds an
+// elements (a fifth to a quarter of the kernel's time: it reads what the product
+// will, from L2).  A tile with a row or column that holds an
 // infinity, that is too small to scale, or whose mean lies more than
 // kSplitSpread binades below its largest (2^-40 of the largest would be more
 // than 2^-25 of an ordinary element) runs on the fp32 instructions instead
-// (fp32_tile).  A NaN needs no care: it is NaN in h, and so in the sums it enters.
+// (fp32_tile).  Where the caller gave a workspace the scan is a launch of its own.
+// A NaN needs no care: it is NaN in h, and so in the sums it enters.
 //
 // Sign.  The f16 instruction drops the low bits of its sum downwards: over a
 // long k the results lie about 1e-7 of their typical size too low (K = 4096),
@@ -39,11 +38,11 @@
 // cores; one barrier per stage, before the stage's last block of rows so that
 // its MFMAs cover the first reads of the next stage.
 //
-// Measured (us; fp32 instructions before, here): NT 8192 x 4096 x 4096 1896, 900
-// (306 TFLOP/s; the matrix cores busy 63% of the cycles at the 1.7 GHz they
-// reach); TN 4096 x 4096 x 8192 1892, 865; NN 2048 x 4096 x 1024 149, 85; TN
-// 1003 x 2050 x 3000 267, 94; NT 1999 x 1531 x 777 104, 54; 64 x NN 1024 x 128 x
-// 1024 268, 158.  Error against 64 bits, of normal data: K = 4096 1.14e-6,
+// Measured (us; fp32 instructions before, scanning in the workgroups, with a scan
+// of its own): NT 8192 x 4096 x 4096 1896, 900, 740 (372 TFLOP/s; the matrix cores
+// busy 63% of the cycles at the 1.7 GHz they reach); TN 4096 x 4096 x 8192 1892,
+// 865, 739; NN 2048 x 4096 x 1024 149, 85, 71; TN 1003 x 2050 x 3000 267, 94, 80; NT
+// 1999 x 1531 x 777 104, 54, 49; 64 x NN 1024 x 128 x 1024 (no workspace) 268, 158.  Error against 64 bits, of normal data: K = 4096 1.14e-6,
 // 7.1e-7; K = 1024 5.7e-7, 3.6e-7.
 //
 // LDS.  An operand stage is h then l, each [row block of 16][64 chunks of 16
@@ -281,8 +280,151 @@ __device__ __forceinline__ void split_scales(SplitScan<R> &S, int *bad) {
     }
 }
 
+// ---- the scan as a launch of its own -------------------------------------------------
+//
+// Where the caller's workspace has room, the operands are scanned once, before
+// the product, instead of by every workgroup: per slice of K, row and chunk of
+// k one SplitRow, the chunks' exact sums added up by the product's workgroups
+// (the same scales and choices as their own scan, and so the same bits).
+// HBM-bound: each operand read once (40 us for 8192 x 4096 and 4096 x 4096).
+struct SplitRow {
+    unsigned top, sum, cnt, pad;
+};
+constexpr int kScanRows = 16;    // k-contiguous: rows per workgroup, four per wave
+constexpr int kScanCols = 64;    // else: columns per workgroup, four per lane, 16 k side by side
+constexpr int kScanChunks = 16;  // at most this many chunks of k
+struct SplitScanArgs {
+    SplitRow *a, *b;             // [slice][chunk][row]; null a: no scan
+    int chunks_a, chunks_b, kc_a, kc_b;  // chunks of k (per slice), and k per chunk
+    int blocks_a, blocks_b;      // workgroups per slice
+};
+
+__device__ __forceinline__ void scan_value(float v, unsigned &top, unsigned &sum, unsigned &cnt) {
+    const unsigned e = __builtin_amdgcn_ubfe(__float_as_uint(v), 23, 8);
+    top = __float_as_uint(fmaxf(__uint_as_float(top), fabsf(v)));
+    sum += e;
+    cnt += min(e, 1u);
+}
+
+template <bool XF>
+__device__ __forceinline__ f4v_t scan_load(const float *p, int have, const XfRegs &xf) {
+    f4v_t v[1];
+    if (have >= 4) v[0] = *reinterpret_cast<const f4u_t *>(p);
+    else v[0] = f4v_t{p[0], have > 1 ? p[1] : 0.0f, have > 2 ? p[2] : 0.0f, 0.0f};
+    if constexpr (XF) xf_regs(xf, v);
+    return v[0];
+}
+
+// Rows of a k-contiguous operand: a wave takes four, 256 k of each at a time.
+template <bool XF>
+__device__ __forceinline__ void scan_rows(const float *X, int rows, int K, int ld, SplitRow *out, int block,
+                                          const XfRegs &xf) {
+    const int lane = threadIdx.x & 63, r0 = block * kScanRows + static_cast<int>(threadIdx.x >> 6) * 4;
+    unsigned top[4] = {}, sum[4] = {}, cnt[4] = {};
+#pragma unroll 2
+    for (int k = lane * 4; k < K; k += 256) {
+        f4v_t v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = scan_load<XF>(X + (size_t)min(r0 + r, rows - 1) * ld + k, K - k, xf);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) scan_value(v[r][c], top[r], sum[r], cnt[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) {
+            top[r] = max(top[r], (unsigned)__shfl_xor((int)top[r], d, 64));
+            sum[r] += __shfl_xor((int)sum[r], d, 64);
+            cnt[r] += __shfl_xor((int)cnt[r], d, 64);
+        }
+        if (lane == r && r0 + r < rows) out[r0 + r] = SplitRow{top[r], sum[r], cnt[r], 0};
+    }
+}
+
+// Columns of the other kind over one chunk of k: 16 lanes take four each, the
+// workgroup's 16 groups of lanes every 16th k.
+template <bool XF>
+__device__ __forceinline__ void scan_cols(const float *X, int rows, int K, int ld, SplitRow *out, int block,
+                                          int chunks, int kc, const XfRegs &xf) {
+    __shared__ unsigned part[3][16][kScanCols];  // top, sum, cnt
+    const int t = threadIdx.x, cl = (t & 15) * 4, kp = t >> 4;
+    const int chunk = block % chunks, c0 = (block / chunks) * kScanCols;
+    const int k1 = min(K, (chunk + 1) * kc), have = rows - c0 - cl;
+    unsigned top[4] = {}, sum[4] = {}, cnt[4] = {};
+    if (have > 0) {
+#pragma unroll 4
+        for (int k = chunk * kc + kp; k < k1; k += 16) {
+            const f4v_t v = scan_load<XF>(X + (size_t)k * ld + c0 + cl, have, xf);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) scan_value(v[c], top[c], sum[c], cnt[c]);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        part[0][kp][cl + c] = top[c];
+        part[1][kp][cl + c] = sum[c];
+        part[2][kp][cl + c] = cnt[c];
+    }
+    __syncthreads();
+    if (t < kScanCols && c0 + t < rows) {
+        SplitRow r{0, 0, 0, 0};
+#pragma unroll
+        for (int w = 0; w < 16; ++w) {
+            r.top = max(r.top, part[0][w][t]);
+            r.sum += part[1][w][t];
+            r.cnt += part[2][w][t];
+        }
+        out[(size_t)chunk * rows + c0 + t] = r;
+    }
+}
+
+template <bool TA, bool TB, bool XF>
+__global__ __launch_bounds__(256) void split_scan(GemmArgs g, SplitScanArgs p) {
+    const int per = p.blocks_a + p.blocks_b;
+    const int slice = static_cast<int>(blockIdx.x) / per;
+    int b = static_cast<int>(blockIdx.x) - slice * per;
+    const int k0 = slice * g.kslice, K = g.kslice > 0 ? min(g.kslice, g.K - k0) : g.K;
+    const XfRegs xf = XF ? xf_load(b < p.blocks_a ? g.xa : g.xb) : XfRegs{};
+    if (b < p.blocks_a) {  // uniform
+        SplitRow *out = p.a + (size_t)slice * p.chunks_a * g.M;
+        const float *X = g.A + (TA ? (size_t)k0 * g.lda : (size_t)k0);
+        if constexpr (TA) scan_cols<XF>(X, g.M, K, g.lda, out, b, p.chunks_a, p.kc_a, xf);
+        else scan_rows<XF>(X, g.M, K, g.lda, out, b, xf);
+    } else {
+        b -= p.blocks_a;
+        SplitRow *out = p.b + (size_t)slice * p.chunks_b * g.N;
+        const float *X = g.B + (TB ? (size_t)k0 : (size_t)k0 * g.ldb);
+        if constexpr (TB) scan_rows<XF>(X, g.N, K, g.ldb, out, b, xf);
+        else scan_cols<XF>(X, g.N, K, g.ldb, out, b, p.chunks_b, p.kc_b, xf);
+    }
+}
+
+// R rows from r0 on of a slice's scan into S.
+template <int R, int NT>
+__device__ __forceinline__ void scan_take(SplitScan<R> &S, const SplitRow *scan, int chunks, int rows, int r0) {
+    for (int r = threadIdx.x; r < R; r += NT) {
+        const SplitRow *p = scan + min(r0 + r, rows - 1);
+        SplitRow v[kScanChunks];  // every load in flight
+#pragma unroll
+        for (int c = 0; c < kScanChunks; ++c) v[c] = p[(size_t)min(c, chunks - 1) * rows];
+        unsigned top = 0, sum = 0, cnt = 0;
+#pragma unroll
+        for (int c = 0; c < kScanChunks; ++c)
+            if (c < chunks) {
+                top = max(top, v[c].top);
+                sum += v[c].sum;
+                cnt += v[c].cnt;
+            }
+        S.top[r] = top;
+        S.sum[r] = sum;
+        S.cnt[r] = cnt;
+    }
+}
+
 template <bool TA, bool TB, int BM, int BN, int WM, int WN, int PF, int EPI, bool CS, bool XF>
-__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split(GemmArgs g, int products) {
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split(GemmArgs g, int products, SplitScanArgs scans) {
     constexpr int NT = 64 * WM * WN;
     if (CS && static_cast<int>(blockIdx.x) >= products) {  // uniform: B's column sums, 16 columns a workgroup
         colsum_strip<NT, XF>(g, (static_cast<int>(blockIdx.x) - products) * kStripCols);
@@ -316,9 +458,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split(GemmArgs g, int pr
         Bp += ob;
         Cp += static_cast<long long>(batch) * g.sc;
     }
-    int K = g.K;
+    int K = g.K, slice = 0;
     if (g.kslice > 0) {  // split K: partial products side by side in C
-        const int slice = bid / g.tiles;
+        slice = bid / g.tiles;
         bid -= slice * g.tiles;
         const int k0 = slice * g.kslice;
         K = min(g.kslice, g.K - k0);
@@ -360,13 +502,20 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split(GemmArgs g, int pr
                     for (int f = 0; f < FUB; ++f) rb[slot][(u - UA) * FUB + f] = SB::load(Bbase + t * bstep, g.ldb, offb, (u - UA) * FUB + f);
                 }
             };
-    // the scan
+    // the scan, or what its own launch found
     const bool edge = (TA && i0 + BM > g.M && (g.M & 3)) || (!TB && j0 + BN > g.N && (g.N & 3));
     const bool tail = nst * kSplitK < K;
     for (int r = threadIdx.x; r < BM; r += NT) sa.top[r] = sa.sum[r] = sa.cnt[r] = 0;
     for (int r = threadIdx.x; r < BN; r += NT) sb.top[r] = sb.sum[r] = sb.cnt[r] = 0;
     if (threadIdx.x == 0) bad = 0;
-    {
+    if (scans.a) {  // uniform
+#pragma unroll
+        for (int u = 0; u < UA + UB; ++u) load(0, u, 0);
+        __syncthreads();
+        scan_take<BM, NT>(sa, scans.a + (size_t)slice * scans.chunks_a * g.M, scans.chunks_a, g.M, i0);
+        scan_take<BN, NT>(sb, scans.b + (size_t)slice * scans.chunks_b * g.N, scans.chunks_b, g.N, j0);
+        __syncthreads();
+    } else {
         float topa[SA::NS] = {}, topb[SB::NS] = {};
         unsigned suma[SA::NS] = {}, sumb[SB::NS] = {}, cnta[SA::NS] = {}, cntb[SB::NS] = {};
         auto scan = [&](f4v_t(&va)[SA::NF], f4v_t(&vb)[SB::NF]) {
@@ -382,7 +531,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split(GemmArgs g, int pr
         constexpr int D = kScanDepth;  // stages in flight
         f4v_t va[D][SA::NF], vb[D][SB::NF];
         auto fetch = [&](int d, int t) {
-            t = min(t, nst - 1);  // past the end: the last stage again, which changes nothing but the counts
+            t = min(t, nst - 1);  // past the end: the last stage again, not scanned
 #pragma unroll
             for (int f = 0; f < SA::NF; ++f) va[d][f] = SA::load(Abase + t * astep, g.lda, offa, f);
 #pragma unroll
@@ -399,7 +548,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split(GemmArgs g, int pr
                         for (int u = 0; u < UA; ++u) SA::mend(va[d], g.M, i0, u);
                     if constexpr (EDGE && !TB)
                         for (int u = 0; u < UB; ++u) SB::mend(vb[d], g.N, j0, u);
-                    scan(va[d], vb[d]);
+                    if (t + d < nst) scan(va[d], vb[d]);  // uniform
                     fetch(d, t + D + d);
                     __builtin_amdgcn_sched_barrier(0);  // the loads before the next stage is waited for
                 }
@@ -418,9 +567,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split(GemmArgs g, int pr
         SA::scan_join(sa, topa, suma, cnta);
         SB::scan_join(sb, topb, sumb, cntb);
         __syncthreads();
-    }
 #pragma unroll
-    for (int u = 0; u < UA + UB; ++u) load(0, u, 0);  // on their way while the scales are found
+        for (int u = 0; u < UA + UB; ++u) load(0, u, 0);  // on their way while the scales are found
+    }
     split_scales<BM, NT>(sa, &bad);
     split_scales<BN, NT>(sb, &bad);
     __syncthreads();
