@@ -227,13 +227,12 @@ __device__ __forceinline__ float tanhf_fdlibm(float x) {
     if (ix < 0x41b00000) {  // |x| < 22
         if (ix == 0) return x;
         if (ix < 0x24000000) return x * (one + x);  // |x| < 2^-55
-        if (ix >= 0x3f800000) {
-            t = expm1f_fdlibm(two * __builtin_fabsf(x));
-            z = one - two / (t + two);
-        } else {
-            t = expm1f_fdlibm(-two * __builtin_fabsf(x));
-            z = -t / (t + two);
-        }
+        // one expm1 and one division for both ranges (a wave's lanes fall in
+        // both: as two branches it ran each of them)
+        const bool large = ix >= 0x3f800000;
+        t = expm1f_fdlibm((large ? two : -two) * __builtin_fabsf(x));
+        z = (large ? two : -t) / (t + two);
+        if (large) z = one - z;
     } else {
         z = one - tiny;
     }
