@@ -212,6 +212,14 @@ int ts_hip_softmax(const float *x, float *y, size_t outer, size_t reduce, size_t
 int ts_hip_broadcast_copy(const float *src, const size_t *src_dims, size_t src_rank, float *out,
                           const size_t *out_dims, size_t out_rank, float scale, int use_scale,
                           void *stream);
+/* ops/{add,sub,mul,div}.rs broadcast paths in one pass (op 0 add, 1 sub, 2 mul,
+ * 3 div): out (out_dims) = a op b, each broadcast NumPy-style, with the bits of
+ * the same op over the operands written out in full.  For div, zero_index as in
+ * ts_hip_div over the flat index from zero_check_start on.  out has fewer than
+ * 2^31 elements (TS_HIP_EINVAL otherwise). */
+int ts_hip_broadcast_binary(int op, const float *a, const size_t *a_dims, size_t a_rank, const float *b,
+                            const size_t *b_dims, size_t b_rank, float *out, const size_t *out_dims,
+                            size_t out_rank, size_t zero_check_start, unsigned long long *zero_index, void *stream);
 /* transform/transpose.rs:156-208 and contiguous.rs:123-157 (the reference's
  * strided view, materialised): out = src (dims, rank) with axes d0 and d1
  * swapped, both row-major; d0 == d1 copies.  A matrix operand of a product

@@ -127,6 +127,8 @@ HIP_SIGNATURES = {
     "ts_hip_softmax": (_c.c_int, [VP, VP, SZ, SZ, SZ, VP]),
     "ts_hip_broadcast_copy": (_c.c_int, [VP, _c.POINTER(SZ), SZ, VP, _c.POINTER(SZ), SZ, _c.c_float,
                                          _c.c_int, VP]),
+    "ts_hip_broadcast_binary": (_c.c_int, [_c.c_int, VP, _c.POINTER(SZ), SZ, VP, _c.POINTER(SZ), SZ, VP,
+                                           _c.POINTER(SZ), SZ, SZ, VP, VP]),
     "ts_hip_reduce_sum": (_c.c_int, [VP, _c.POINTER(SZ), SZ, _c.c_uint, VP, _c.c_float, _c.c_int, VP]),
     "ts_hip_transpose": (_c.c_int, [VP, _c.POINTER(SZ), SZ, SZ, SZ, VP, VP]),
     "ts_hip_map_jit_mode": (_c.c_int, [_c.c_int]),

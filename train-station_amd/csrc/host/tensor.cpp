@@ -133,6 +133,34 @@ Tensor bcast_to(const float *src, const std::vector<size_t> &src_dims, const std
     return out;
 }
 
+// out (dims) = a op b, each broadcast to it: in one pass, or past that kernel's
+// 2^31 elements with the operands that need it written out first
+// (broadcast_shapes, broadcasting.rs:362-407).
+Tensor bcast_binary(const float *a, const std::vector<size_t> &a_dims, const float *b, const std::vector<size_t> &b_dims,
+                    const std::vector<size_t> &dims, int op) {
+    if (product(dims) >= (size_t(1) << 31)) {
+        Tensor ab, bb;
+        if (a_dims != dims) {
+            ab = bcast_to(a, a_dims, dims);
+            a = ab.dev();
+        }
+        if (b_dims != dims) {
+            bb = bcast_to(b, b_dims, dims);
+            b = bb.dev();
+        }
+        return same_shape(a, b, dims, op);
+    }
+    Tensor out = Tensor::new_uninit(dims);
+    const size_t n = out.size();
+    if (n)
+        launch(KernelClass::Elementwise, 4.0 * n + 4.0 * product(a_dims) + 4.0 * product(b_dims), "broadcast op", [&] {
+            return ts_hip_broadcast_binary(op, a, a_dims.data(), a_dims.size(), b, b_dims.data(), b_dims.size(),
+                                           out.dev_mut(), dims.data(), dims.size(), tail32(n),
+                                           op == 3 ? Runtime::get().zero_index() : nullptr, S());
+        });
+    return out;
+}
+
 // Sum of x over the axes in `mask` into a tensor of `out_dims` (the keepdim
 // layout, possibly with the size-1 axes removed: the same element order).
 Tensor reduce_axes(const float *x, const std::vector<size_t> &dims, unsigned mask, std::vector<size_t> out_dims,
@@ -193,13 +221,12 @@ bool is_row_broadcast(const std::vector<size_t> &full, const std::vector<size_t>
 }
 
 // go (full shape) op broadcast(x): x itself when it has the full shape, the
-// row-broadcast kernel for a [N] vector over [B, N], else x materialised.
+// row-broadcast kernel for a [N] vector over [B, N], else the general one.
 Tensor with_bcast(const Tensor &go, const SavedTensor &x, int op) {
     if (x.dims == go.dims()) return same_shape(go.dev(), x.ptr(), go.dims(), op);
     if (is_row_broadcast(go.dims(), x.dims))
         return row_bcast(go.dev(), x.ptr(), go.dims()[0], go.dims()[1], op, false);
-    Tensor xb = bcast_to(x.ptr(), x.dims, go.dims());
-    return same_shape(go.dev(), xb.dev(), go.dims(), op);
+    return bcast_binary(go.dev(), go.dims(), x.ptr(), x.dims, go.dims(), op);
 }
 
 // softmax's [outer, reduce, inner] view of an axis
@@ -1370,20 +1397,7 @@ Tensor Tensor::binary(const Tensor &o, GradFn::Kind kind) const {
     } else if (is_row_broadcast(o.dims_, dims_)) {
         out = row_bcast(o.dev(), dev(), o.dims_[0], o.dims_[1], op, true);
     } else {
-        // broadcast_shapes (broadcasting.rs:362-407): materialise the operands
-        // that need it, then the same-shape kernel
-        const std::vector<size_t> full = broadcast_dims(dims_, o.dims_);
-        Tensor ab, bb;
-        const float *pa = dev(), *pb = o.dev();
-        if (dims_ != full) {
-            ab = bcast_to(dev(), dims_, full);
-            pa = ab.dev();
-        }
-        if (o.dims_ != full) {
-            bb = bcast_to(o.dev(), o.dims_, full);
-            pb = bb.dev();
-        }
-        out = same_shape(pa, pb, full, op);
+        out = bcast_binary(dev(), dims_, o.dev(), o.dims_, broadcast_dims(dims_, o.dims_), op);
     }
     if ((requires_grad_ || o.requires_grad_) && is_grad_enabled()) {
         GradFn fn{kind};
