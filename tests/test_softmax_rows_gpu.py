@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("rows,cols", [
     (130, 9), (70, 10), (9, 33), (9, 64), (8, 65), (17, 128), (7, 129), (8, 256), (3, 257), (5, 512), (4, 513), (6, 1000),
-    (1, 1024), (5, 1025), (3, 2048), (5, 2049), (5, 4097), (3, 8192), (3, 8193), (2, 16385), (1, 32768), (2, 32769)])
+    (1, 1024), (5, 1025), (3, 2048), (5, 2049), (5, 4097), (3, 8192), (3, 8193), (2, 16385), (1, 32768), (2, 32769),
+    (2050, 2049), (2049, 3001), (3601, 4097), (1801, 8200), (901, 16385), (9, 40000)])
 def test_softmax_rows(rows, cols):
     from gpu_util import Dev, hip, hip_check, sync
 
