@@ -243,3 +243,24 @@ def test_split_batched(ta, tb, batches, M, N, K):
         fine = np.isfinite(want)
         assert np.array_equal(np.isfinite(got[i]), fine)
         assert np.all(np.abs(got[i] - want)[fine] <= (K * 2.0 ** -24 * mag)[fine])
+
+
+@pytest.mark.parametrize("rank", [0, 1])
+@pytest.mark.parametrize("ta,tb,M,N,K", [(0, 0, 2048, 1408, 640), (0, 1, 769, 641, 16001), (1, 0, 999, 777, 1001)])
+def test_split_batch_of_one(rank, ta, tb, M, N, K):
+    # sizes whose 2-D product splits K: the batched call has no room for the partial products
+    from gpu_util import Dev, hip, hip_check, sync
+    from train_station_amd._ffi import SZ
+
+    print(f"[split, batch of one] ta={ta} tb={tb} {M}x{N}x{K} rank={rank}", flush=True)
+    a, b = normal((K, M) if ta else (M, K), 45), normal((N, K) if tb else (K, N), 46)
+    da, db, dc = Dev.of(a), Dev.of(b), Dev.of(np.full(M * N, np.nan, np.float32))
+    dims, zero = (SZ * 1)(1), (SZ * 1)(0)
+    hip_check(hip.ts_hip_gemm_batched(ta, tb, M, N, K, da.ptr, a.shape[1], db.ptr, b.shape[1], dc.ptr, N, rank, dims,
+                                      zero, zero, M * N, None), "batched")
+    sync()
+    got = dc.get((M, N))
+    assert np.all(np.isfinite(got))
+    i, j, want, mag = _sample(a, b, ta, tb, np.random.default_rng(1), M, N)
+    # one fp32 addition per term at most
+    assert np.all(np.abs(got[np.ix_(i, j)] - want) <= K * 2.0 ** -24 * mag)

@@ -2096,8 +2096,9 @@ extern "C" int ts_hip_gemm_batched(int trans_a, int trans_b, size_t M, size_t N,
         g.sb[k] = static_cast<long long>(b_batch_strides[k]);
     }
     g.sc = static_cast<long long>(c_batch_stride);
+    // this call has no workspace for slices of K, which a batch of one can ask for
     const SplitPlan plan = split_plan(M, N, K, batches);
-    if (plan.on && A && B && lda >= (trans_a ? M : K) && ldb >= (trans_b ? K : N) && split_lds_ok(lda, ldb, ldc)) {
+    if (plan.on && plan.slices == 1 && A && B && lda >= (trans_a ? M : K) && ldb >= (trans_b ? K : N) && split_lds_ok(lda, ldb, ldc)) {
         gemm_operands(g, M, N, K, A, lda, B, ldb, C, ldc);
         return launch_split(plan, trans_a, trans_b, g, static_cast<unsigned>(batches), nullptr, nullptr,
                             as_stream(stream));
