@@ -264,3 +264,30 @@ def test_split_batch_of_one(rank, ta, tb, M, N, K):
     i, j, want, mag = _sample(a, b, ta, tb, np.random.default_rng(1), M, N)
     # one fp32 addition per term at most
     assert np.all(np.abs(got[np.ix_(i, j)] - want) <= K * 2.0 ** -24 * mag)
+
+
+@pytest.mark.parametrize("ta,tb", [(1, 0), (0, 0), (1, 1)])
+@pytest.mark.parametrize("left", [1, 2, 3])
+def test_split_last_rows_stay_inside(ta, tb, left):
+    # a last tile of one to three rows, K in whole stages, scanned by the workgroups: what lies behind a
+    # row-contiguous operand is not read (an infinity there would send the tile to the fp32 instructions)
+    from gpu_util import Dev, hip, hip_check, sync
+    from train_station_amd._ffi import SZ
+
+    M = N = 1152 + left
+    K = 1024
+    print(f"[split, last rows] ta={ta} tb={tb} 2 x {M}x{N}x{K}", flush=True)
+    a, b = normal((K, M) if ta else (M, K), 43), normal((N, K) if tb else (K, N), 44)
+    dims, shared = (SZ * 1)(2), (SZ * 1)(0)
+    out = []
+    for behind in (0.0, np.inf):
+        tail = np.full(8, behind, np.float32)
+        da, db = Dev.of(np.concatenate([a.ravel(), tail])), Dev.of(np.concatenate([b.ravel(), tail]))
+        dc = Dev(2 * M * N)
+        hip_check(hip.ts_hip_gemm_batched(ta, tb, M, N, K, da.ptr, a.shape[1], db.ptr, b.shape[1], dc.ptr, N, 1, dims,
+                                          shared, shared, M * N, None), "batched")
+        sync()
+        out.append(dc.get((2, M, N)))
+    assert_bits_equal(out[1], out[0], "zeros and infinities behind the operands")
+    i, j, want, mag = _sample(a, b, ta, tb, np.random.default_rng(1), M, N)
+    assert np.all(np.abs(out[0][1][np.ix_(i, j)] - want) <= (4 + 6 * (K + 31) // 32) * 2.0 ** -24 * mag)

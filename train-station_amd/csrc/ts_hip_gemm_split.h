@@ -137,7 +137,11 @@ struct SplitStage {
             half = (n / (R / 4)) & 1;
         }
     }
-    // byte offset of a unit's first float4 from the tile's first row and k
+    // The row the offsets start from: the tile's first, or where fewer than four
+    // are left of the operand its fourth last (not KC), so that no float4 ends
+    // past the operand.
+    static __device__ __forceinline__ int first(int rows, int r0) { return KC ? r0 : min(r0, rows - 4); }
+    // byte offset of a unit's first float4 from row first() and the stage's first k
     static __device__ __forceinline__ void offsets(unsigned (&off)[U], int ld, int rows, int r0) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -145,7 +149,7 @@ struct SplitStage {
             coords(u, row, q, half);
             if (KC) off[u] = static_cast<unsigned>(min(row, rows - 1 - r0)) * static_cast<unsigned>(ld) * 4u + 16u * q;
             else off[u] = static_cast<unsigned>(16 * half + 4 * q) * static_cast<unsigned>(ld) * 4u +
-                          4u * static_cast<unsigned>(max(0, min(row, rows - 4 - r0)));
+                          4u * static_cast<unsigned>(min(row, rows - 4 - first(rows, r0)));
         }
     }
     // float4 number f of a whole stage
@@ -175,7 +179,7 @@ struct SplitStage {
     static __device__ __forceinline__ void mend(f4v_t (&reg)[NF], int rows, int r0, int u) {
         int row, q, half;
         coords(u, row, q, half);
-        const int s = row - max(0, min(row, rows - 4 - r0));  // 1..3 for it, 4 and more for those past the operand
+        const int s = row - min(row, rows - 4 - r0);  // 1..3 for it, 4 and more for those past the operand
 #pragma unroll
         for (int f = 4 * u; f < 4 * u + 4; ++f) {
             const f4v_t v = reg[f];
@@ -485,8 +489,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split(GemmArgs g, int pr
     unsigned offa[SA::U], offb[SB::U];
     SA::offsets(offa, g.lda, g.M, i0);
     SB::offsets(offb, g.ldb, g.N, j0);
-    const float *Abase = TA ? Ap + i0 : Ap + (size_t)i0 * g.lda;
-    const float *Bbase = TB ? Bp + (size_t)j0 * g.ldb : Bp + j0;
+    const int ai = SA::first(g.M, i0), bj0 = SB::first(g.N, j0);
+    const float *Abase = TA ? Ap + ai : Ap + (size_t)ai * g.lda;
+    const float *Bbase = TB ? Bp + (size_t)bj0 * g.ldb : Bp + bj0;
     const size_t astep = TA ? (size_t)kSplitK * g.lda : kSplitK, bstep = TB ? kSplitK : (size_t)kSplitK * g.ldb;
 
             constexpr int UA = SA::U, UB = SB::U, FUA = SA::NF / UA, FUB = SB::NF / UB;
