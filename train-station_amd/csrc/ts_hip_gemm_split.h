@@ -494,19 +494,21 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split(GemmArgs g, int pr
     const float *Bbase = TB ? Bp + (size_t)bj0 * g.ldb : Bp + bj0;
     const size_t astep = TA ? (size_t)kSplitK * g.lda : kSplitK, bstep = TB ? kSplitK : (size_t)kSplitK * g.ldb;
 
-            constexpr int UA = SA::U, UB = SB::U, FUA = SA::NF / UA, FUB = SB::NF / UB;
-            const int nst = K / kSplitK;  // whole stages, at least one
+    constexpr int UA = SA::U, UB = SB::U, FUA = SA::NF / UA, FUB = SB::NF / UB;
+    const int nst = K / kSplitK;  // whole stages, at least one
     f4v_t ra[PF][SA::NF], rb[PF][SB::NF];
     auto load = [&](int slot, int u, int t) {  // unit u (A's, then B's) of stage t
-                t = min(t, nst - 1);  // past the end: the last stage again, never used
-                if (u < UA) {
-    #pragma unroll
-                    for (int f = 0; f < FUA; ++f) ra[slot][u * FUA + f] = SA::load(Abase + t * astep, g.lda, offa, u * FUA + f);
-                } else {
-    #pragma unroll
-                    for (int f = 0; f < FUB; ++f) rb[slot][(u - UA) * FUB + f] = SB::load(Bbase + t * bstep, g.ldb, offb, (u - UA) * FUB + f);
-                }
-            };
+        t = min(t, nst - 1);  // past the end: the last stage again, never used
+        if (u < UA) {
+#pragma unroll
+            for (int f = 0; f < FUA; ++f)
+                ra[slot][u * FUA + f] = SA::load(Abase + t * astep, g.lda, offa, u * FUA + f);
+        } else {
+#pragma unroll
+            for (int f = 0; f < FUB; ++f)
+                rb[slot][(u - UA) * FUB + f] = SB::load(Bbase + t * bstep, g.ldb, offb, (u - UA) * FUB + f);
+        }
+    };
     // the scan, or what its own launch found
     const bool edge = (TA && i0 + BM > g.M && (g.M & 3)) || (!TB && j0 + BN > g.N && (g.N & 3));
     const bool tail = nst * kSplitK < K;
