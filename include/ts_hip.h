@@ -384,23 +384,25 @@ int ts_hip_matmul(const float *a, const float *b, float *c, size_t m, size_t n, 
  *   trans_b == 1: B(k,j) = B[j*ldb + k]   (B stored [N][ldb], i.e. B^T view)
  *   C(i,j) = C[i*ldc + j]
  * fp32 inputs and accumulation.  Products of 2.2e9 operations and more (1.5e9
- * where M, N or K is no multiple of 4; not the untransposed ones that the
- * 16x16x4 kernel below takes) run on the f16 matrix cores: each value, scaled into range by its row of op(A) or
- * column of op(B), as the sum of two f16 values (within 2^-24 of itself or
- * 2^-40 of its row's largest), three f16 products summed in fp32 -- closer to
- * the exact product than the fp32 instructions.  Output tiles whose rows or
- * columns hold an infinity or spread too far for that, and smaller products,
- * run on the fp32 instructions (v_mfma_f32_16x16x4_f32 when M and N are
- * multiples of 256, K of 32 and the grid has a 256x256 tile per CU; else
- * v_mfma_f32_32x32x2_f32).  The kinds add k in different groupings, so a
- * product's last bits depend on which it takes; every entry point below takes
- * the same one for the same shape, layout and alignment.  M, N, K and
+ * where M, N or K is no multiple of 4; not the untransposed ones whose B has
+ * 2^23 elements or more, nor those that split K or have N <= 16) run on the
+ * bf16 matrix cores: each value is exactly the sum of three bf16 values, and of
+ * their nine products six are summed in fp32 (the others are below 2^-24 of the
+ * term together).  Each element of C is then within (20 + K/16) 2^-24 of the
+ * exact one, times its sum of |a| |b|, whatever the operands' ranges.  Output
+ * tiles with a sum that is not finite there (an infinity or a NaN in an operand,
+ * values past 2^111, sums past 2^95), and the other products, run on the fp32
+ * instructions (v_mfma_f32_16x16x4_f32 when M and N are multiples of 256, K of
+ * 32 and the grid has a 256x256 tile per CU; else v_mfma_f32_32x32x2_f32),
+ * within K 2^-24.  The kinds add k in different groupings, so a product's last
+ * bits depend on which it takes; every entry point below takes the same one for
+ * the same shape, layout and alignment (a batch counts as part of the shape).
+ * M, N, K and
  * the leading dimensions must be below 2^31 (TS_HIP_EINVAL otherwise).  For
  * few output tiles with a long K (e.g. M = 32, K = 784) the call splits K and
  * takes a temporary of up to 16*M*N floats from the stream-ordered allocator
  * (hipMallocAsync / hipFreeAsync on `stream`); where that allocator is
- * unavailable it runs unsplit, as does a product on the f16 matrix cores while
- * a graph is recorded. */
+ * unavailable it runs unsplit. */
 int ts_hip_gemm(int trans_a, int trans_b, size_t M, size_t N, size_t K, const float *A,
                 size_t lda, const float *B, size_t ldb, float *C, size_t ldc, void *stream);
 
@@ -408,7 +410,7 @@ int ts_hip_gemm(int trans_a, int trans_b, size_t M, size_t N, size_t K, const fl
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  Same arguments,
  * kernels and results (bit for bit) as ts_hip_gemm; a split product's
- * temporary comes from a fixed device array of 9 * 2^20 floats (36 MiB) that each
+ * temporary comes from a fixed device array of 2^21 floats (8 MiB) that each
  * device holds for the life of the process, which every split this device
  * can choose fits (a product needing more returns TS_HIP_ESCRATCH).  The
  * array is shared by all calls on a device: calls that overlap on one device
@@ -416,10 +418,9 @@ int ts_hip_gemm(int trans_a, int trans_b, size_t M, size_t N, size_t K, const fl
 int ts_hip_gemm_noalloc(int trans_a, int trans_b, size_t M, size_t N, size_t K, const float *A,
                         size_t lda, const float *B, size_t ldb, float *C, size_t ldc, void *stream);
 
-/* Floats of workspace a product can use: the temporary of a K split over
- * workgroups (what ts_hip_gemm takes from the stream-ordered allocator), and on
- * the f16 matrix cores a scan of the operands, without which its workgroups
- * scan (the same result, slower).  0 when the product M x N x K uses none. */
+/* Floats of workspace a split product needs (the temporary ts_hip_gemm takes
+ * from the stream-ordered allocator for few output tiles with a long K):
+ * 0 when the product M x N x K is not split. */
 size_t ts_hip_gemm_workspace_floats(size_t M, size_t N, size_t K);
 
 /* The same product with the elementwise ops that follow it fused into the
@@ -435,8 +436,7 @@ size_t ts_hip_gemm_workspace_floats(size_t M, size_t N, size_t K);
  * Bit-identical to ts_hip_gemm followed by ts_hip_bias_add, ts_hip_relu and
  * ts_hip_relu_backward(mask, C, C).  A split product (see
  * ts_hip_gemm_workspace_floats) uses `workspace` (device, at least that many
- * floats; with fewer, one on the f16 matrix cores does without and the others
- * return TS_HIP_EWORKSPACE) as its temporary, so the call allocates
+ * floats; TS_HIP_EWORKSPACE if fewer) as its temporary, so the call allocates
  * nothing and can be recorded into a HIP graph; with workspace == NULL it
  * allocates as ts_hip_gemm does. */
 int ts_hip_gemm_fused(int trans_a, int trans_b, size_t M, size_t N, size_t K, const float *A, size_t lda,

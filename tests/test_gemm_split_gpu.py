@@ -1,14 +1,12 @@
-"""Products on the f16 matrix cores (2.2e9 operations and more, 1.5e9 of ragged sizes): every layout at
-the edges of the tiles, of the k stages and of the split K, odd leading
-dimensions and addresses, the rows that are left to the fp32 instructions, and
-one result from every entry point.
+"""Products on the bf16 matrix cores (2.2e9 operations and more, 1.5e9 of ragged sizes): every layout at
+the edges of the tiles and of the stages of k, odd leading dimensions and addresses, operands of any range,
+the tiles that are left to the fp32 instructions, and one result from every entry point.
 
-Bound, per element: the two factors of a term are each within 2^-24 of
-themselves (or 2^-40 of their row's largest, at most 2^-25 of a row that is
-split), the smallest partial product left out is below 2^-24 of it, and three
-sums of 32 terms are added to a running sum per 32 k, each within two roundings
-of 2^-24: 4 + 2 * 3 * K / 32 units of 2^-24 of sum |a| |b|; the fp32 tiles add
-one term at a time, K units."""
+Bound, per element, in units of 2^-24 of sum |a| |b|: the pieces' products left out are below 1; six
+instructions add a stage of 16 k from zero, each dropping less than 2 of that stage's sum |a| |b|: 12 in all;
+a stage joins the running sum, and the four groups' sums each other, with one rounding: K / 16 + 2 + 4; and
+the result takes one more when its scale is taken back (to the subnormal grid where it is that small).
+The fp32 instructions' bound, one rounding a term, is K: the larger for K >= 64."""
 from __future__ import annotations
 
 import numpy as np
@@ -18,9 +16,14 @@ from conftest import assert_bits_equal, normal
 
 pytestmark = pytest.mark.gpu
 
+
+def _bound(K, mag):
+    return (20 + K / 16) * 2.0 ** -24 * mag + 2.0 ** -149
+
+
 # (trans_a, trans_b, M, N, K, operand pitch pad, operand offset in floats)
 CASES = [
-    (0, 0, 4224, 4224, 256, 0, 0),      # 256x256 tiles
+    (0, 0, 4224, 4224, 256, 0, 0),      # 128x128 tiles, two a CU
     (0, 1, 4096, 4096, 256, 0, 0),
     (1, 0, 4096, 4096, 256, 0, 0),
     (1, 1, 4096, 4096, 256, 0, 0),
@@ -28,19 +31,25 @@ CASES = [
     (0, 1, 4095, 4091, 255, 3, 1),
     (1, 0, 4093, 4094, 224, 0, 1),
     (1, 1, 4089, 4090, 193, 1, 3),
-    (0, 0, 2048, 1408, 640, 0, 0),      # 128x128 tiles, K in two
+    (0, 0, 2048, 1408, 640, 0, 0),      # 128x128 tiles, two groups
     (0, 1, 2049, 1409, 641, 0, 0),
     (1, 0, 2051, 1411, 643, 1, 0),
     (1, 1, 2050, 1410, 642, 0, 1),
-    (0, 0, 2049, 4097, 200, 0, 0),      # K whole
+    (0, 0, 2049, 4097, 200, 0, 0),      # one group
     (0, 1, 2050, 4099, 191, 1, 1),
     (1, 0, 2051, 4098, 224, 0, 3),
     (1, 1, 2047, 4095, 231, 0, 0),
-    (0, 0, 769, 641, 16001, 0, 0),      # few tiles: K split, its last slice short
+    (0, 0, 769, 641, 13001, 0, 0),      # 64x64 tiles, four groups, the last one's stages short
     (0, 1, 771, 643, 16383, 0, 1),
     (1, 0, 897, 513, 16000, 3, 0),
     (1, 1, 641, 770, 20011, 0, 0),
-    (0, 0, 100, 16384, 1024, 0, 0),     # one row of tiles, most of it used
+    (0, 0, 100, 8130, 1030, 0, 0),      # one row of 64x128 tiles and a part
+    (0, 1, 96, 12000, 1004, 0, 1),
+    (1, 0, 1531, 777, 1999, 0, 0),      # 64x128 tiles, two groups, one stage more for the first
+    (1, 1, 1999, 777, 1063, 1, 0),
+    (0, 1, 4097, 67, 4001, 0, 0),       # fewer columns than the wider tiles have
+    (0, 0, 4160, 4160, 64, 0, 0),       # the fewest k
+    (0, 1, 5001, 4161, 79, 0, 0),
     (1, 0, 25000, 1000, 67, 0, 0),      # few k
     (0, 0, 1280, 1280, 672, 0, 0),      # the smallest
     (1, 0, 999, 777, 1001, 0, 0),
@@ -85,19 +94,102 @@ def test_split_products(ta, tb, M, N, K, pad, off):
         assert np.all(np.isnan(out[:, N:])), "the output pitch's padding was written"
     i, j, want, mag = _sample(a, b, ta, tb, np.random.default_rng(1), M, N)
     err = np.abs(got[np.ix_(i, j)] - want)
-    assert np.all(err <= (4 + 6 * (K + 31) // 32) * 2.0 ** -24 * mag)
-    # and closer than one rounding a term would leave it, over all
-    assert np.sqrt(np.mean(err ** 2)) <= 0.5 * np.sqrt(K) * 2.0 ** -24 * np.sqrt(np.mean(want ** 2))
+    assert np.all(err <= _bound(K, mag))
+    # and closer than one rounding in two terms, as the fp32 instructions take them, leaves it
+    assert np.sqrt(np.mean(err ** 2)) <= 0.3 * np.sqrt(K / 2) * 2.0 ** -24 * np.sqrt(np.mean(want ** 2)) + 2.0 ** -149
+
+
+# Values of every range in one row: kind, and what it asks of A (M x K) and B (K x N).
+def _ranges(kind, A, B, rng):
+    K = A.shape[1]
+    sel = np.zeros(K, bool)
+    share, e = {"a quarter at 2^-45": (0.25, -45), "a fifth at 2^-41": (0.2, -41), "a tenth at 2^-60": (0.1, -60),
+                "an eighth at 2^-120": (0.125, -120)}.get(kind, (0, 0))
+    if share:  # a few small columns of A, the only ones that B's rows meet
+        sel[rng.choice(K, int(share * K), replace=False)] = True
+        return np.where(sel, A * np.float32(2.0) ** e, A), np.where(sel[:, None], B, np.float32(0))
+    if kind.startswith("opposite halves"):
+        s = np.float32(2.0) ** int(kind.split("^")[1])
+        half = np.arange(K) % 2 == 0
+        return np.where(half, A * s, A), np.where(half[:, None], B, B * s)
+    if kind == "term-balanced":
+        s = (np.float32(2.0) ** rng.integers(-60, 61, K)).astype(np.float32)
+        return A * s, B / s[:, None]
+    if kind == "rows of mixed magnitude":
+        return A * (np.float32(2.0) ** rng.integers(-40, 41, A.shape)).astype(np.float32), B
+    if kind == "both tiny":  # products on the subnormal grid
+        return A * np.float32(2.0 ** -66), B * np.float32(2.0 ** -66)
+    if kind == "subnormal and huge":
+        return (A * np.float32(2.0 ** -126)) * np.float32(2.0 ** -12), B * np.float32(2.0 ** 90)
+    assert kind == "past the stages' scale"
+    return A * np.float32(2.0 ** 115), B * np.float32(2.0 ** -110)
+
+
+RANGES = ["a quarter at 2^-45", "a fifth at 2^-41", "a tenth at 2^-60", "an eighth at 2^-120", "opposite halves 2^-20",
+          "opposite halves 2^-22", "term-balanced", "rows of mixed magnitude", "both tiny", "subnormal and huge",
+          "past the stages' scale"]
+# one size of each tile: 64x64, 64x128, 128x128 by two groups and by one
+TILES = [(769, 770, 1280), (1100, 1300, 1024), (2049, 1409, 643), (3001, 2050, 512)]
 
 
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
-@pytest.mark.parametrize("M,N,K", [(4224, 4224, 128), (2048, 1409, 640), (769, 769, 16001)])
-def test_split_rows_left_to_fp32(ta, tb, M, N, K):
+@pytest.mark.parametrize("kind", RANGES)
+def test_split_values_of_any_range(ta, tb, kind):
+    from gpu_util import Dev, hip, hip_check, sync
+
+    for M, N, K in TILES:
+        print(f"[split, {kind}] ta={ta} tb={tb} {M}x{N}x{K}", flush=True)
+        rng = np.random.default_rng(K)
+        A, B = _ranges(kind, normal((M, K), 41), normal((K, N), 42), rng)
+        a, b = (np.ascontiguousarray(A.T) if ta else A), (np.ascontiguousarray(B.T) if tb else B)
+        da, db, dc = Dev.of(a), Dev.of(b), Dev(M * N)
+        hip_check(hip.ts_hip_gemm(ta, tb, M, N, K, da.ptr, a.shape[1], db.ptr, b.shape[1], dc.ptr, N, None), "gemm")
+        sync()
+        i, j, want, mag = _sample(a, b, ta, tb, rng, M, N)
+        got = dc.get((M, N))[np.ix_(i, j)]
+        # (what the fp32 instructions have is within one rounding a term; products below the normal range
+        # round to the subnormal grid there)
+        tol = K * 2.0 ** -24 * mag + K * 2.0 ** -149 if kind.startswith("past") else _bound(K, mag)
+        assert np.all(np.abs(got - want) <= tol), (kind, M, N, K)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_split_exact_products(ta, tb):
+    # products that are fp32 values come out as they are: by a permutation (values of any magnitude) and of
+    # whole numbers; a sum of nothing is +0
+    from gpu_util import Dev, hip, hip_check, sync
+
+    for M, N, K in TILES + [(1500, 1024, 1024)]:
+        print(f"[split, exact] ta={ta} tb={tb} {M}x{N}x{K}", flush=True)
+        rng = np.random.default_rng(M)
+        A = normal((M, K), 47) * (np.float32(2.0) ** rng.integers(-100, 90, (M, K))).astype(np.float32)
+        cols = rng.integers(0, K, N)
+        P = np.zeros((K, N), np.float32)
+        P[cols, np.arange(N)] = 1
+        whole = rng.integers(-4096, 4097, (M, K)).astype(np.float32), rng.integers(-3, 4, (K, N)).astype(np.float32)
+        # rows of zeros of either sign, and terms that cancel to nothing
+        Z, B = normal((M, K), 48), normal((K, N), 49)
+        Z[5], Z[6] = 0.0, -0.0
+        Z[7, 1::2] = Z[7, 0:K - K % 2:2]
+        Z[7, K - K % 2:] = 0
+        B[1:K:2] = -B[0:K - 1:2]
+        for X, Y, want, rows in ((A, P, A[:, cols], slice(None)), (*whole, whole[0] @ whole[1], slice(None)),
+                                 (Z, B, np.zeros((3, N), np.float32), slice(5, 8))):
+            x, y = (np.ascontiguousarray(X.T) if ta else X), (np.ascontiguousarray(Y.T) if tb else Y)
+            da, db, dc = Dev.of(x), Dev.of(y), Dev(M * N)
+            hip_check(hip.ts_hip_gemm(ta, tb, M, N, K, da.ptr, x.shape[1], db.ptr, y.shape[1], dc.ptr, N, None), "gemm")
+            sync()
+            assert_bits_equal(dc.get((M, N))[rows], want, f"{M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(4224, 4224, 128), (2048, 1409, 640), (1999, 777, 1063), (769, 769, 16001)])
+def test_split_tiles_left_to_fp32(ta, tb, M, N, K):
     # op(A)'s rows: 3 an infinity, 130 a NaN, 200 the type's lowest value beside ordinary ones that meet
     # zeros, 257 one outlier of 2^60, 300 tiny values, 301 subnormals, 400 zeros; op(B)'s column 5 an infinity
     from gpu_util import Dev, hip, hip_check, sync
 
-    print(f"[split, fp32 rows] ta={ta} tb={tb} {M}x{N}x{K}", flush=True)
+    print(f"[split, fp32 tiles] ta={ta} tb={tb} {M}x{N}x{K}", flush=True)
     A, B = normal((M, K), 33), normal((K, N), 34)
     A[3, 7] = np.inf
     A[130, 9] = np.nan
@@ -124,16 +216,19 @@ def test_split_rows_left_to_fp32(ta, tb, M, N, K):
     fine = np.isfinite(f32)
     # one term at a time in fp32; products of subnormals round to the subnormal grid
     tol = K * 2.0 ** -24 * mag + K * 2.0 ** -149
-    assert np.all(np.abs(g.astype(np.float64) - want)[fine] <= tol[fine])
-    assert not np.any(got[400][np.arange(N) != 5])
+    assert np.all(np.abs(g[fine].astype(np.float64) - want[fine]) <= tol[fine])
+    zeros = got[400][np.arange(N) != 5]
+    assert not np.any(zeros) and not np.any(np.signbit(zeros))
 
 
 @pytest.mark.parametrize("ta,tb,M,N,K", [(0, 0, 4224, 4224, 96), (1, 0, 4100, 4100, 96), (0, 1, 2050, 1410, 642),
-                                         (1, 0, 2048, 1408, 640), (1, 0, 769, 769, 16383)])
+                                         (1, 0, 2048, 1408, 640), (1, 0, 769, 769, 16383), (1, 0, 1531, 777, 1999),
+                                         (0, 0, 1024, 4096, 2048), (0, 0, 520, 4100, 2050)])  # the last two: fp32
 def test_split_entry_points(oracle, ta, tb, M, N, K):
-    # the plain, the workspace, the allocation-free and the column-sum call: one product, and the
-    # epilogue the separate kernels' bits
+    # the plain, the fused, the allocation-free, the column-sum and the batched call: one product, without a
+    # workspace, and the epilogue the separate kernels' bits
     from gpu_util import Dev, hip, hip_check, sync
+    from train_station_amd._ffi import SZ
 
     print(f"[split entries] ta={ta} tb={tb} {M}x{N}x{K}", flush=True)
     a, b = normal((K, M) if ta else (M, K), 35), normal((N, K) if tb else (K, N), 36)
@@ -143,9 +238,7 @@ def test_split_entry_points(oracle, ta, tb, M, N, K):
     hip_check(hip.ts_hip_gemm(ta, tb, M, N, K, da.ptr, lda, db.ptr, ldb, ref.ptr, N, None), "gemm")
     sync()
     want = ref.get()
-    need = hip.ts_hip_gemm_workspace_floats(M, N, K)
-    assert 0 < need <= 9 << 20
-    ws = Dev(need)
+    assert hip.ts_hip_gemm_workspace_floats(M, N, K) == 0
 
     def same(what):
         sync()
@@ -154,9 +247,14 @@ def test_split_entry_points(oracle, ta, tb, M, N, K):
 
     hip_check(hip.ts_hip_gemm_noalloc(ta, tb, M, N, K, da.ptr, lda, db.ptr, ldb, new.ptr, N, None), "noalloc")
     same("noalloc")
-    hip_check(hip.ts_hip_gemm_fused(ta, tb, M, N, K, da.ptr, lda, db.ptr, ldb, None, 0, None, new.ptr, N, ws.ptr, need,
+    hip_check(hip.ts_hip_gemm_fused(ta, tb, M, N, K, da.ptr, lda, db.ptr, ldb, None, 0, None, new.ptr, N, None, 0,
                                     None), "fused")
-    same("workspace")
+    same("fused")
+    dims, zero = (SZ * 1)(1), (SZ * 1)(0)
+    for rank in (0, 1):
+        hip_check(hip.ts_hip_gemm_batched(ta, tb, M, N, K, da.ptr, lda, db.ptr, ldb, new.ptr, N, rank, dims, zero,
+                                          zero, M * N, None), "batched")
+        same(f"a batch of one, rank {rank}")
     if not tb:
         cs = Dev(N)
         cneed = hip.ts_hip_gemm_colsum_workspace_floats(ta, M, N, K)
@@ -166,56 +264,12 @@ def test_split_entry_points(oracle, ta, tb, M, N, K):
         same("colsum")
         assert_bits_equal(cs.get(), oracle.sum_dim0_chunked(b), "column sums vs the oracle's order")
     hip_check(hip.ts_hip_gemm_fused(ta, tb, M, N, K, da.ptr, lda, db.ptr, ldb, bias.ptr, 1, mask.ptr, new.ptr, N,
-                                    ws.ptr, need, None), "fused epilogue")
+                                    None, 0, None), "fused epilogue")
     hip_check(hip.ts_hip_bias_add(ref.ptr, bias.ptr, ref.ptr, M, N, 0, None), "bias")
     hip_check(hip.ts_hip_relu(ref.ptr, ref.ptr, M * N, None), "relu")
     hip_check(hip.ts_hip_relu_backward(mask.ptr, ref.ptr, ref.ptr, M * N, None), "mask")
     sync()
     assert_bits_equal(new.get(), ref.get(), "epilogue")
-    new.put(np.full(M * N, np.nan, np.float32))
-    hip_check(hip.ts_hip_gemm_fused(ta, tb, M, N, K, da.ptr, lda, db.ptr, ldb, None, 0, None, new.ptr, N, None, 0,
-                                    None), "no workspace")
-    same("the stream-ordered allocator's workspace")
-    # one float fewer: the operands scanned by the workgroups, the same scales; one float in all: a K that was split
-    # (fewer tiles than CUs) whole, not an error
-    new.put(np.full(M * N, np.nan, np.float32))
-    args = (ta, tb, M, N, K, da.ptr, lda, db.ptr, ldb, None, 0, None, new.ptr, N, ws.ptr)
-    hip_check(hip.ts_hip_gemm_fused(*args, need - 1, None), "a smaller workspace")
-    same("a smaller workspace")
-    hip_check(hip.ts_hip_gemm_fused(*args, 1, None), "a small workspace")
-    if M >= 4096:
-        same("a small workspace")
-    else:
-        sync()
-        _, _, _, mag = _sample(a, b, ta, tb, np.random.default_rng(1), M, N)
-        assert np.max(np.abs(new.get().astype(np.float64) - want)) <= (8 + 12 * K / 32) * 2.0 ** -24 * np.max(mag)
-
-
-def test_split_scans_agree():
-    # rows and columns of every kind (wide ranges, zeros, infinities, subnormals): the scan's own launch and the
-    # workgroups' scan leave the same tiles to the fp32 instructions
-    from gpu_util import Dev, hip, hip_check, sync
-
-    rng = np.random.default_rng(7)
-    for ta, tb, M, N, K in [(0, 1, 2049, 1025, 1003), (1, 0, 1025, 2051, 1001), (0, 0, 4100, 4100, 131),
-                            (1, 1, 1100, 1300, 1999)]:
-        print(f"[split scans] ta={ta} tb={tb} {M}x{N}x{K}", flush=True)
-        A, B = normal((M, K), 41), normal((K, N), 42)
-        A[rng.integers(0, M, 3)] *= np.float32(2.0) ** rng.integers(-60, 60, K).astype(np.float32)
-        B[:, rng.integers(0, N, 3)] *= np.float32(2.0) ** rng.integers(-13, 13, (K, 1)).astype(np.float32)
-        A[M - 1, K - 1] = np.inf
-        A[5] = 0
-        A[6] = 1e-42
-        B[0, N - 1] = 3e38
-        a, b = (np.ascontiguousarray(A.T) if ta else A), (np.ascontiguousarray(B.T) if tb else B)
-        da, db, c1, c2 = Dev.of(a), Dev.of(b), Dev(M * N), Dev(M * N)
-        need = hip.ts_hip_gemm_workspace_floats(M, N, K)
-        ws = Dev(need)
-        for c, n in ((c1, need), (c2, need - 1)):
-            hip_check(hip.ts_hip_gemm_fused(ta, tb, M, N, K, da.ptr, a.shape[1], db.ptr, b.shape[1], None, 0, None,
-                                            c.ptr, N, ws.ptr, n, None), "fused")
-        sync()
-        assert_bits_equal(c1.get(), c2.get(), f"{M}x{N}x{K}")
 
 
 @pytest.mark.parametrize("ta,tb,batches,M,N,K", [(0, 0, 6, 1024, 1000, 300), (0, 1, 64, 256, 256, 512),
@@ -227,7 +281,7 @@ def test_split_batched(ta, tb, batches, M, N, K):
     print(f"[split batched] ta={ta} tb={tb} {batches} x {M}x{N}x{K}", flush=True)
     a = normal((batches,) + ((K, M) if ta else (M, K)), 39)
     b = normal((N, K) if tb else (K, N), 40)  # shared by the batch
-    a[1, 3, 5] = np.inf  # one tile of one batch to the fp32 instructions
+    a[1, 3, 5] = np.inf  # one row of tiles of one batch to the fp32 instructions
     da, db, dc = Dev.of(a), Dev.of(b), Dev(batches * M * N)
     dims, sa, sb = (SZ * 1)(batches), (SZ * 1)(M * K), (SZ * 1)(0)
     hip_check(hip.ts_hip_gemm_batched(ta, tb, M, N, K, da.ptr, a.shape[2], db.ptr, b.shape[1], dc.ptr, N, 1, dims, sa,
@@ -242,35 +296,14 @@ def test_split_batched(ta, tb, batches, M, N, K):
             mag = np.abs(A) @ np.abs(B)
         fine = np.isfinite(want)
         assert np.array_equal(np.isfinite(got[i]), fine)
-        assert np.all(np.abs(got[i] - want)[fine] <= (K * 2.0 ** -24 * mag)[fine])
-
-
-@pytest.mark.parametrize("rank", [0, 1])
-@pytest.mark.parametrize("ta,tb,M,N,K", [(0, 0, 2048, 1408, 640), (0, 1, 769, 641, 16001), (1, 0, 999, 777, 1001)])
-def test_split_batch_of_one(rank, ta, tb, M, N, K):
-    # sizes whose 2-D product splits K: the batched call has no room for the partial products
-    from gpu_util import Dev, hip, hip_check, sync
-    from train_station_amd._ffi import SZ
-
-    print(f"[split, batch of one] ta={ta} tb={tb} {M}x{N}x{K} rank={rank}", flush=True)
-    a, b = normal((K, M) if ta else (M, K), 45), normal((N, K) if tb else (K, N), 46)
-    da, db, dc = Dev.of(a), Dev.of(b), Dev.of(np.full(M * N, np.nan, np.float32))
-    dims, zero = (SZ * 1)(1), (SZ * 1)(0)
-    hip_check(hip.ts_hip_gemm_batched(ta, tb, M, N, K, da.ptr, a.shape[1], db.ptr, b.shape[1], dc.ptr, N, rank, dims,
-                                      zero, zero, M * N, None), "batched")
-    sync()
-    got = dc.get((M, N))
-    assert np.all(np.isfinite(got))
-    i, j, want, mag = _sample(a, b, ta, tb, np.random.default_rng(1), M, N)
-    # one fp32 addition per term at most
-    assert np.all(np.abs(got[np.ix_(i, j)] - want) <= K * 2.0 ** -24 * mag)
+        assert np.all(np.abs(got[i][fine] - want[fine]) <= (K * 2.0 ** -24 * mag)[fine])
 
 
 @pytest.mark.parametrize("ta,tb", [(1, 0), (0, 0), (1, 1)])
 @pytest.mark.parametrize("left", [1, 2, 3])
 def test_split_last_rows_stay_inside(ta, tb, left):
-    # a last tile of one to three rows, K in whole stages, scanned by the workgroups: what lies behind a
-    # row-contiguous operand is not read (an infinity there would send the tile to the fp32 instructions)
+    # a last tile of one to three rows, K in whole stages: what lies behind an operand is not read (an
+    # infinity there would send the tile to the fp32 instructions)
     from gpu_util import Dev, hip, hip_check, sync
     from train_station_amd._ffi import SZ
 
@@ -290,4 +323,4 @@ def test_split_last_rows_stay_inside(ta, tb, left):
         out.append(dc.get((2, M, N)))
     assert_bits_equal(out[1], out[0], "zeros and infinities behind the operands")
     i, j, want, mag = _sample(a, b, ta, tb, np.random.default_rng(1), M, N)
-    assert np.all(np.abs(out[0][1][np.ix_(i, j)] - want) <= (4 + 6 * (K + 31) // 32) * 2.0 ** -24 * mag)
+    assert np.all(np.abs(out[0][1][np.ix_(i, j)] - want) <= _bound(K, mag))

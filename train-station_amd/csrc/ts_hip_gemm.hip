@@ -1626,26 +1626,13 @@ struct GemmPlan {
     size_t split_floats = 0;
     size_t part_floats = 0;
     bool cs_kernel = false;  // the product's kernels write the column sums
-    SplitPlan f16;           // on the f16 matrix cores (its partial products counted in split_floats)
-    void unslice() {
-        if (f16.slices < 2) return;
-        f16.slices = 1;
-        f16.kslice = 0;
-        f16.partial_floats = 0;
-        drop_scan();
-    }
-    // Without a scan of its own (that launch needs a workspace from the caller).
-    void drop_scan() {
-        f16.scan_floats = 0;
-        if (f16.on) split_floats = f16.partial_floats;
-    }
-    size_t scan_offset() const { return (f16.partial_floats + 3) & ~size_t(3); }
+    SplitPlan split;         // on the bf16 matrix cores (no workspace; column sums as the fp32 tiles)
     size_t part_offset() const { return (split_floats + 1) & ~size_t(1); }
     size_t total() const { return part_floats ? part_offset() + part_floats : split_floats; }
 };
 
-// f16_ok false: without the f16 matrix cores (leading dimensions past their reach).
-static GemmPlan gemm_plan(int trans_a, int trans_b, size_t M, size_t N, size_t K, bool colsum, bool f16_ok = true) {
+// split_ok false: without the bf16 matrix cores (leading dimensions past their reach).
+static GemmPlan gemm_plan(int trans_a, int trans_b, size_t M, size_t N, size_t K, bool colsum, bool split_ok = true) {
     GemmPlan p;
     if (M == 0 || N == 0 || K == 0) return p;
     p.skinny = skinny(N);
@@ -1661,23 +1648,7 @@ static GemmPlan gemm_plan(int trans_a, int trans_b, size_t M, size_t N, size_t K
     // (sized whenever the grid could take that kernel: alignment is not known here)
     const bool dma_cs = p.cs_kernel && !p.narrow && big_grid(M, N, 1);
     p.part_floats = colsum && (!p.cs_kernel || dma_cs) ? 2 * colsum_chunk_count(K) * N : 0;
-    // The untransposed products with an exact tiling stay on the fp32 kernel
-    // (at 93% of those instructions' peak).  They are a network's forward
-    // products, whose rounding decides the units of a relu that lie within it
-    // of zero: with six layers of 4096 units on the f16 cores the first
-    // layer's weights were 5e-3 from the fp32 kernels' after two steps (any
-    // two roundings of the forward products differ so; the results are no
-    // further from 64 bits), with this 1e-4.  Shallower and smaller networks
-    // showed 1e-3 and less either way.
-    const bool fp32 = !trans_a && !trans_b && M % 256 == 0 && N % 256 == 0 && K % 32 == 0 && big_grid(M, N, 1);
-    if (f16_ok && !fp32 && !p.skinny && !p.narrow) p.f16 = split_plan(M, N, K, 1);
-    if (p.f16.on) {
-        // their 128 x 128 tiles append the fp32 tiles' column strips; past
-        // those a column-sum pass follows
-        p.cs_kernel = colsum && trans_a && !trans_b && p.f16.tile == 128;
-        p.split_floats = p.f16.scan_floats ? p.scan_offset() + p.f16.scan_floats : p.f16.partial_floats;
-        p.part_floats = colsum && !p.cs_kernel ? 2 * colsum_chunk_count(K) * N : 0;
-    }
+    if (split_ok && !p.skinny && !p.narrow && p.slices == 1) p.split = split_plan(trans_a, trans_b, M, N, K, 1);
     return p;
 }
 
@@ -1720,30 +1691,17 @@ static bool xf_from(const ts_hip_operand_xf *x, OperandXf &out) {
     return true;
 }
 
-// The operands and sizes of a product in the kernels' terms.
+// The operands and sizes of a product in the bf16 kernels' terms.
 static void gemm_operands(GemmArgs &g, size_t M, size_t N, size_t K, const float *A, size_t lda, const float *B,
                           size_t ldb, float *C, size_t ldc) {
     g.A = A; g.B = B; g.C = C;
     g.M = static_cast<int>(M); g.N = static_cast<int>(N); g.K = static_cast<int>(K);
     g.lda = static_cast<int>(lda); g.ldb = static_cast<int>(ldb); g.ldc = static_cast<int>(ldc);
-    bool strides4 = true;
-    for (int k = 0; k < g.batch_rank; ++k) strides4 = strides4 && g.sa[k] % 4 == 0 && g.sb[k] % 4 == 0;
-    g.vec = vec_operands(A, lda, B, ldb) && strides4;
 }
 
-// Whether work issued on s is being recorded into a graph.
-static bool capturing(hipStream_t s) {
-    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &c) != hipSuccess) {
-        (void)hipGetLastError();
-        return true;
-    }
-    return c != hipStreamCaptureStatusNone;
-}
-
-// Leading dimensions whose lane offsets fit the f16 kernels' 32 bits.
+// Leading dimensions whose lane offsets fit the bf16 kernels' 32 bits.
 static bool split_lds_ok(size_t lda, size_t ldb, size_t ldc) {
-    const size_t lim = size_t(1) << 22;
+    const size_t lim = size_t(1) << 24;
     return lda < lim && ldb < lim && ldc < (size_t(1) << 31);
 }
 
@@ -1772,15 +1730,9 @@ static int gemm_plain(int trans_a, int trans_b, size_t M, size_t N, size_t K, co
         return st;
     }
     if (!A || !B || lda < (trans_a ? M : K) || ldb < (trans_b ? K : N)) return TS_HIP_EINVAL;
-    GemmPlan plan = gemm_plan(trans_a, trans_b, M, N, K, colsum != nullptr, split_lds_ok(lda, ldb, ldc));
-    hipStream_t st = as_stream(stream);
-    // A product on the f16 matrix cores without room for its scan (no workspace
-    // of the caller's, or a smaller one) scans in its workgroups, and without
-    // room for its slices (a smaller one yet, or none while a graph is
-    // recorded) runs whole.
-    if (plan.f16.on && (!ws || ws_floats < plan.total() || (reinterpret_cast<uintptr_t>(ws) & 15))) plan.drop_scan();
-    if (plan.f16.slices > 1 && (ws ? ws_floats < plan.total() : capturing(st))) plan.unslice();
+    const GemmPlan plan = gemm_plan(trans_a, trans_b, M, N, K, colsum != nullptr, split_lds_ok(lda, ldb, ldc));
     const size_t need = plan.total();
+    hipStream_t st = as_stream(stream);
     float *W = ws;
     bool owned = false;
     if (need && ws && (ws_floats < need || (plan.part_floats && (reinterpret_cast<uintptr_t>(ws) & 7u))))
@@ -1792,7 +1744,6 @@ static int gemm_plain(int trans_a, int trans_b, size_t M, size_t N, size_t K, co
         } else {
             (void)hipGetLastError();
             W = nullptr;
-            plan.unslice();
             // no stream-ordered memory: an MFMA split runs unsplit; the rest
             // needs memory, and the allocator's error is returned
             // (hipErrorOutOfMemory when the device is full)
@@ -1821,7 +1772,7 @@ static int gemm_plain(int trans_a, int trans_b, size_t M, size_t N, size_t K, co
         g.colsum = colsum;
         g.colsum_part = part;
         status = launch_skinny(trans_a, trans_b, M, N, K, A, lda, B, ldb, C, ldc, g, W, stream);
-    } else if (plan.f16.on) {
+    } else if (plan.split.on) {
         GemmArgs g{};
         g.bias = bias;
         g.mask = mask;
@@ -1830,7 +1781,7 @@ static int gemm_plain(int trans_a, int trans_b, size_t M, size_t N, size_t K, co
         if (xb) g.xb = *xb;
         gemm_operands(g, M, N, K, A, lda, B, ldb, C, ldc);
         if (plan.cs_kernel) g.colsum = colsum;
-        status = launch_split(plan.f16, trans_a, trans_b, g, 1, W, plan.f16.scan_floats ? W + plan.scan_offset() : nullptr, st);
+        status = launch_split(plan.split, trans_a, trans_b, g, 1, st);
         if (status == TS_HIP_OK && colsum && !plan.cs_kernel)
             status = launch_colsum(B, nullptr, K, N, ldb, colsum, reinterpret_cast<float *>(part), plan.part_floats,
                                    stream);
@@ -1889,10 +1840,8 @@ extern "C" int ts_hip_gemm(int trans_a, int trans_b, size_t M, size_t N, size_t 
 
 // ---- allocation-free form --------------------------------------------------
 //
-// ts_hip_gemm_noalloc takes a product's workspace from this fixed device
-// array instead of the stream-ordered allocator.  A product on the f16 matrix
-// cores asks for at most 2^23 floats of partial products and 2^20 of its scan
-// (36 MiB; split_plan chooses no other).  An MFMA split runs only
+// ts_hip_gemm_noalloc takes the split-K temporary from this fixed device
+// array instead of the stream-ordered allocator.  An MFMA split runs only
 // while 4 * (64x64 tiles) < CUs with slices * tiles <= 2 * CUs, so it never
 // needs more than 2 * CUs * 64 * 64 floats: 2^21 (8 MiB) on the 256 CUs of an
 // MI355X; a skinny split (N <= 16) has fewer 64-row groups than CUs and at
@@ -1900,7 +1849,7 @@ extern "C" int ts_hip_gemm(int trans_a, int trans_b, size_t M, size_t N, size_t 
 // of the process.  Calls that overlap on one device (several streams) share
 // it and race; the split slices are fully written before they are read, so
 // nothing needs clearing between calls.
-static constexpr size_t kScratchFloats = 9 * (size_t(1) << 20) + 64;
+static constexpr size_t kScratchFloats = size_t(1) << 21;
 static __device__ __align__(256) float scratch[kScratchFloats];
 
 namespace tship {
@@ -1943,10 +1892,7 @@ extern "C" int ts_hip_gemm_noalloc(int trans_a, int trans_b, size_t M, size_t N,
 }
 
 extern "C" size_t ts_hip_gemm_workspace_floats(size_t M, size_t N, size_t K) {
-    // the layout that takes most: NT products run on the f16 matrix cores where
-    // NN ones of an exact tiling do not
-    const size_t nn = gemm_plan(0, 0, M, N, K, false).total(), nt = gemm_plan(0, 1, M, N, K, false).total();
-    return nn > nt ? nn : nt;
+    return gemm_plan(0, 0, M, N, K, false).total();
 }
 
 extern "C" int ts_hip_gemm_fused(int trans_a, int trans_b, size_t M, size_t N, size_t K, const float *A,
@@ -2096,12 +2042,11 @@ extern "C" int ts_hip_gemm_batched(int trans_a, int trans_b, size_t M, size_t N,
         g.sb[k] = static_cast<long long>(b_batch_strides[k]);
     }
     g.sc = static_cast<long long>(c_batch_stride);
-    // this call has no workspace for slices of K, which a batch of one can ask for
-    const SplitPlan plan = split_plan(M, N, K, batches);
-    if (plan.on && plan.slices == 1 && A && B && lda >= (trans_a ? M : K) && ldb >= (trans_b ? K : N) && split_lds_ok(lda, ldb, ldc)) {
+    const SplitPlan plan =  // a batch of one as ts_hip_gemm
+        batches == 1 ? gemm_plan(trans_a, trans_b, M, N, K, false).split : split_plan(trans_a, trans_b, M, N, K, batches);
+    if (plan.on && A && B && lda >= (trans_a ? M : K) && ldb >= (trans_b ? K : N) && split_lds_ok(lda, ldb, ldc)) {
         gemm_operands(g, M, N, K, A, lda, B, ldb, C, ldc);
-        return launch_split(plan, trans_a, trans_b, g, static_cast<unsigned>(batches), nullptr, nullptr,
-                            as_stream(stream));
+        return launch_split(plan, trans_a, trans_b, g, static_cast<unsigned>(batches), as_stream(stream));
     }
     return gemm_launch(trans_a, trans_b, M, N, K, A, lda, B, ldb, C, ldc, g, batches, stream);
 }

@@ -122,7 +122,7 @@ struct GemmArgs {
     // they go.  Null: none.
     float *colsum;
     double *colsum_part;
-    int kslice;  // skinny and split-K f16 products: k rows per slice
+    int kslice;  // skinny products: k rows per slice
     // operand transforms (register-staged tiles, the narrow and one-k-tile
     // kernels and the column strips apply them; the others take none)
     OperandXf xa, xb;
@@ -493,24 +493,16 @@ __device__ __forceinline__ void fp32_tile(const GemmArgs &g, const float *Ap, co
 template <int BM>
 constexpr int prefetch_tiles() { return BM >= 256 ? 1 : 4; }
 
-// ---- products on the f16 matrix cores (ts_hip_gemm_split.hip) ---------------------
+// ---- products on the bf16 matrix cores (ts_hip_gemm_split.hip) --------------------
 
-// What such a product takes: 256 x 256 or 128 x 128 tiles, and K in `slices` of
-// kslice (0: whole), whose partial products need partial_floats of workspace.
-// With scan_floats more the operands are scanned by a launch of their own, the
-// faster (the same result without).
+// Whether a product takes them (every entry point asks here), its tile (bm x bn
+// of C per workgroup) and the groups of waves that share a tile's K.
 struct SplitPlan {
     bool on = false;
-    int tile = 0;
-    int slices = 1;
-    int kslice = 0;
-    size_t partial_floats = 0, scan_floats = 0;
+    int bm = 0, bn = 0, groups = 1;
 };
-SplitPlan split_plan(size_t M, size_t N, size_t K, size_t batches);
-// The product (a split one by its slices' partial products in `partial`); g as for the
-// fp32 kernels (its colsum is written for 128 x 128 tiles, not for 256 x 256).
-// scan: scan_floats of workspace (16-byte aligned), or null.
-int launch_split(const SplitPlan &plan, int ta, int tb, GemmArgs g, unsigned batches, float *partial, float *scan,
-                 hipStream_t s);
+SplitPlan split_plan(int trans_a, int trans_b, size_t M, size_t N, size_t K, size_t batches);
+// The product; g as for the fp32 kernels (no sum_out).
+int launch_split(const SplitPlan &plan, int ta, int tb, GemmArgs g, unsigned batches, hipStream_t s);
 
 }  // namespace tship
