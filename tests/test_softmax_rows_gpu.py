@@ -47,3 +47,38 @@ def test_softmax_rows_without_a_value():
     hip_check(hip.ts_hip_softmax(dx.ptr, dy.ptr, 5, 100, 1, None), "softmax")
     sync()
     assert_bits_equal(dy.get(x.shape), O.softmax(x, 1), "softmax")
+
+
+def test_softmax_more_rows_than_a_grid_holds():
+    # 2^29 rows of 10 columns and some take 2^32 threads, more than a launch: the rows at both ends and
+    # where the launches meet, forward and backward
+    from gpu_util import Dev, hip, hip_check, sync
+
+    rows, cols = (1 << 29) + 100, 10
+    print(f"[softmax rows] {rows}x{cols}", flush=True)
+    n = rows * cols
+    dx, dy, dgi = Dev(n), Dev(n), Dev(n)  # 21.5 GB each
+    hip_check(hip.ts_hip_fill(dx.ptr, 0.0, n, None), "fill")
+    hip_check(hip.ts_hip_fill(dgi.ptr, 7.0, n, None), "fill")
+    sync()
+    first = ((1 << 32) - 1) // 64 * 8  # rows of the first launch
+    windows = [(0, 20), (first - 20, 40), (rows - 20, 20)]
+    values = [normal((k, cols), 60 + i, 3.0) for i, (_, k) in enumerate(windows)]
+
+    def put(d, r, v):
+        hip_check(hip.ts_hip_memcpy(d.ptr + 4 * r * cols, v.ctypes.data, v.size, 0), "H2D")
+
+    def get(d, r, k):
+        out = np.empty((k, cols), np.float32)
+        hip_check(hip.ts_hip_memcpy(out.ctypes.data, d.ptr + 4 * r * cols, out.size, 1), "D2H")
+        return out
+
+    for (r, _), v in zip(windows, values):
+        put(dx, r, v)
+    hip_check(hip.ts_hip_softmax(dx.ptr, dy.ptr, rows, cols, 1, None), "softmax")
+    hip_check(hip.ts_hip_softmax_backward(dy.ptr, dx.ptr, dgi.ptr, rows, cols, 1, None), "softmax_backward")
+    sync()
+    for (r, k), v in zip(windows, values):
+        y = O.softmax(v, 1)
+        assert_bits_equal(get(dy, r, k), y, f"softmax, rows from {r}")
+        assert_bits_equal(get(dgi, r, k), O.softmax_bwd(y, v, 1), f"softmax_backward, rows from {r}")

@@ -363,11 +363,17 @@ __global__ __launch_bounds__(kLongBlock) void softmax_long_bwd(const float *__re
 // workgroup's registers end.
 constexpr size_t kRowsMinCols = 10, kRegMaxCols = 32768, kRowsMaxCols = size_t(1) << 30;
 
+// In as many launches as the rows take: a grid holds fewer than 2^32 threads
+// (2^29 rows of 10 columns are that many).
 template <bool FWD, int RW, int CPL, int W>
 static void launch_rows_as(const float *a, const float *b, float *out, size_t rows, int cols, hipStream_t s) {
-    const dim3 grid(static_cast<unsigned>((rows + RW - 1) / RW)), block(64 * W);
-    if constexpr (FWD) launch((softmax_rows_fwd<RW, CPL, W>), grid, block, 0, s, a, out, rows, cols);
-    else launch((softmax_rows_bwd<RW, CPL, W>), grid, block, 0, s, a, b, out, rows, cols);
+    constexpr size_t kRows = ((size_t(1) << 32) - 1) / (64 * W) * RW;
+    for (size_t r = 0; r < rows; r += kRows) {
+        const size_t n = rows - r < kRows ? rows - r : kRows, at = r * cols;
+        const dim3 grid(static_cast<unsigned>((n + RW - 1) / RW)), block(64 * W);
+        if constexpr (FWD) launch((softmax_rows_fwd<RW, CPL, W>), grid, block, 0, s, a + at, out + at, n, cols);
+        else launch((softmax_rows_bwd<RW, CPL, W>), grid, block, 0, s, a + at, b + at, out + at, n, cols);
+    }
 }
 
 // Past 4096 columns a CU's registers hold 4 rows, 2 or 1, and a round of them
