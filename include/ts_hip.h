@@ -390,8 +390,8 @@ int ts_hip_matmul(const float *a, const float *b, float *c, size_t m, size_t n, 
  * their nine products six are summed in fp32 (the others are below 2^-24 of the
  * term together).  Each element of C is then within (20 + K/16) 2^-24 of the
  * exact one, times its sum of |a| |b|, whatever the operands' ranges.  Output
- * tiles with a sum that is not finite there (an infinity or a NaN in an operand,
- * values past 2^111, sums past 2^95), and the other products, run on the fp32
+ * tiles with an infinity in their operands, values past 2^111 or sums past 2^95,
+ * and the other products, run on the fp32
  * instructions (v_mfma_f32_16x16x4_f32 when M and N are multiples of 256, K of
  * 32 and the grid has a 256x256 tile per CU; else v_mfma_f32_32x32x2_f32),
  * within K 2^-24.  The kinds add k in different groupings, so a product's last

@@ -121,13 +121,15 @@ def _ranges(kind, A, B, rng):
         return A * np.float32(2.0 ** -66), B * np.float32(2.0 ** -66)
     if kind == "subnormal and huge":
         return (A * np.float32(2.0 ** -126)) * np.float32(2.0 ** -12), B * np.float32(2.0 ** 90)
+    if kind == "past the stages' sums":
+        return A * np.float32(2.0 ** 70), B * np.float32(2.0 ** 45)
     assert kind == "past the stages' scale"
     return A * np.float32(2.0 ** 115), B * np.float32(2.0 ** -110)
 
 
 RANGES = ["a quarter at 2^-45", "a fifth at 2^-41", "a tenth at 2^-60", "an eighth at 2^-120", "opposite halves 2^-20",
           "opposite halves 2^-22", "term-balanced", "rows of mixed magnitude", "both tiny", "subnormal and huge",
-          "past the stages' scale"]
+          "past the stages' scale", "past the stages' sums"]
 # one size of each tile: 64x64, 64x128, 128x128 by two groups and by one
 TILES = [(769, 770, 1280), (1100, 1300, 1024), (2049, 1409, 643), (3001, 2050, 512)]
 
@@ -219,6 +221,34 @@ def test_split_tiles_left_to_fp32(ta, tb, M, N, K):
     assert np.all(np.abs(g[fine].astype(np.float64) - want[fine]) <= tol[fine])
     zeros = got[400][np.arange(N) != 5]
     assert not np.any(zeros) and not np.any(np.signbit(zeros))
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("scale", [0, 50])
+def test_split_nan_operands(ta, tb, scale):
+    # NaNs alone stay on the bf16 instructions (scale 0); beside sums past their range (2^100) the tile does not
+    from gpu_util import Dev, hip, hip_check, sync
+
+    for M, N, K in TILES:
+        print(f"[split, NaN] ta={ta} tb={tb} {M}x{N}x{K} scale={scale}", flush=True)
+        s = np.float32(2.0 ** scale)
+        A, B = normal((M, K), 51) * s, normal((K, N), 52) * s
+        rows, cols = [0, M // 2, M - 1], [5, N - 1]
+        for r in rows:
+            A[r, (7 * r) % K] = np.nan
+        B[K - 1, cols] = np.nan
+        a, b = (np.ascontiguousarray(A.T) if ta else A), (np.ascontiguousarray(B.T) if tb else B)
+        da, db, dc = Dev.of(a), Dev.of(b), Dev(M * N)
+        hip_check(hip.ts_hip_gemm(ta, tb, M, N, K, da.ptr, a.shape[1], db.ptr, b.shape[1], dc.ptr, N, None), "gemm")
+        sync()
+        got = dc.get((M, N))
+        nan = np.zeros((M, N), bool)
+        nan[rows], nan[:, cols] = True, True
+        assert np.array_equal(np.isnan(got), nan)
+        i, j, want, mag = _sample(np.nan_to_num(a), np.nan_to_num(b), ta, tb, np.random.default_rng(1), M, N)
+        fine = ~nan[np.ix_(i, j)]
+        tol = K * 2.0 ** -24 * mag if scale else _bound(K, mag)
+        assert np.all(np.abs(got[np.ix_(i, j)][fine] - want[fine]) <= tol[fine])
 
 
 @pytest.mark.parametrize("ta,tb,M,N,K", [(0, 0, 4224, 4224, 96), (1, 0, 4100, 4100, 96), (0, 1, 2050, 1410, 642),
@@ -324,3 +354,40 @@ def test_split_last_rows_stay_inside(ta, tb, left):
     assert_bits_equal(out[1], out[0], "zeros and infinities behind the operands")
     i, j, want, mag = _sample(a, b, ta, tb, np.random.default_rng(1), M, N)
     assert np.all(np.abs(out[0][1][np.ix_(i, j)] - want) <= _bound(K, mag))
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("side", ["a", "b"])
+def test_split_transformed_operands(ta, tb, side):
+    # an elementwise chain applied as the operand is loaded: the bits of a buffer that holds its values, also
+    # where a tile is left to the fp32 instructions, and with the column sums
+    import ctypes
+
+    from gpu_util import Dev, hip, hip_check, sync
+    from test_xf_gpu import OTHER, _apply, _xf
+
+    for M, N, K in TILES:
+        print(f"[split, transformed] ta={ta} tb={tb} {side} {M}x{N}x{K}", flush=True)
+        assert hip.ts_hip_gemm_takes_xf(ta, tb, M, N, K, 0) == 1
+        a, b = normal((K, M) if ta else (M, K), 53), normal((N, K) if tb else (K, N), 54)
+        a.flat[7], b.flat[11], b.flat[-1] = np.inf, np.nan, 2.0 ** 100  # the last one squared: an infinity
+        ax, bx = (_apply(a, OTHER), b) if side == "a" else (a, _apply(b, OTHER))
+        x = ctypes.byref(_xf(OTHER))
+        xa, xb = (x, None) if side == "a" else (None, x)
+        lda, ldb = a.shape[1], b.shape[1]
+        da, db, dax, dbx = Dev.of(a), Dev.of(b), Dev.of(ax), Dev.of(bx)
+        got, want = Dev(M * N), Dev(M * N)
+        hip_check(hip.ts_hip_gemm_fused_xf(ta, tb, M, N, K, da.ptr, lda, xa, db.ptr, ldb, xb, None, 0, None, got.ptr,
+                                           N, None, 0, None), "fused_xf")
+        hip_check(hip.ts_hip_gemm(ta, tb, M, N, K, dax.ptr, lda, dbx.ptr, ldb, want.ptr, N, None), "gemm")
+        sync()
+        assert_bits_equal(got.get(), want.get(), f"{M}x{N}x{K}")
+        if ta and not tb:
+            cs_got, cs_want = Dev(N), Dev(N)
+            hip_check(hip.ts_hip_gemm_colsum_xf(ta, M, N, K, da.ptr, lda, xa, db.ptr, ldb, xb, got.ptr, N, cs_got.ptr,
+                                                None, 0, None), "colsum_xf")
+            hip_check(hip.ts_hip_gemm_colsum(ta, M, N, K, dax.ptr, lda, dbx.ptr, ldb, want.ptr, N, cs_want.ptr, None,
+                                             0, None), "colsum")
+            sync()
+            assert_bits_equal(got.get(), want.get(), f"{M}x{N}x{K} with column sums")
+            assert_bits_equal(cs_got.get(), cs_want.get(), "column sums")

@@ -14,9 +14,10 @@
 //
 // Range.  Both operands are staged times 2^16 (exact) and the finished sums
 // taken back by 2^-32 (ldexp, one rounding): the pieces of the smallest
-// subnormals are then bf16 values too.  Where a sum is not finite -- an infinity
-// or a NaN in an operand, a value past 2^111 or a sum past 2^95 -- the tile is
-// computed again on the fp32 instructions (fp32_tile) and has their result.
+// subnormals are then bf16 values too.  A NaN is NaN in h, and so in the sums it
+// enters.  Where a sum is not finite for another reason -- an infinity in an
+// operand, a value past 2^111 or a sum past 2^95 -- the tile is computed again on
+// the fp32 instructions (fp32_tile) and has their result.
 //
 // Sums.  Six instructions add up the pieces' products of 16 k from zero, and the
 // vector units add that to the running sum, so it is rounded once per 16 k
@@ -146,6 +147,35 @@ struct SplitStage {
         }
         return v;
     }
+    // the largest magnitude among a thread's values of the tile's rows (NaNs aside)
+    template <bool XF>
+    static __device__ __forceinline__ float largest(const float *base, int thread, int ld, size_t step, int K,
+                                                    const XfRegs &xf) {
+        const unsigned off = offset(thread, ld);
+        float m = 0.0f;
+        auto take = [&](f4v_t (&v)[NF]) {
+            if constexpr (XF) xf_regs(xf, v);
+#pragma unroll
+            for (int f = 0; f < NF; ++f)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) m = fmaxf(m, fabsf(v[f][c]));
+        };
+        int k = 0;
+#pragma unroll 4
+        for (; k + kSplitK <= K; k += kSplitK, base += step) {
+            f4v_t v[NF];
+#pragma unroll
+            for (int f = 0; f < NF; ++f) v[f] = load(base, ld, off, f);
+            take(v);
+        }
+        if (k < K) {
+            f4v_t v[NF];
+#pragma unroll
+            for (int f = 0; f < NF; ++f) v[f] = load_edge(base, thread, ld, 0, K - k, f);
+            take(v);
+        }
+        return m;
+    }
     // unit u's values times sc, split, into a stage
     static __device__ __forceinline__ void store(char *S, int thread, const f4v_t (&reg)[NF], float sc, int u) {
         int row, part;
@@ -188,6 +218,7 @@ __global__ __launch_bounds__(64 * WM * WN * KG, KG > 2 ? KG : 2) void gemm_split
     __shared__ __attribute__((aligned(16))) char lds[KG * kGroupLds];
     static_assert(KG * kGroupLds >= (KG - 1) * BM * BN * 4, "room for the groups' sums");
     __shared__ int bad;
+    __shared__ unsigned top[2];
 
     const float *Ap = g.A, *Bp = g.B;
     float *Cp = g.C;
@@ -394,7 +425,9 @@ __global__ __launch_bounds__(64 * WM * WN * KG, KG > 2 ? KG : 2) void gemm_split
                 for (int r = 0; r < 16; ++r) acc[n / FN][n % FN][r] += sums[((k * FM * FN + n) * 16 + r) * NT + thread];
     }
 
-    // a sum that is not finite: the tile again on the fp32 instructions
+    // A sum that is not finite: it stays if it can only be a NaN of the operands'
+    // (their finite values too small for a sum to pass the range), else the tile
+    // again on the fp32 instructions.
     {
         float worst = 0.0f;  // NaN * 0 and inf * 0 stay NaN
 #pragma unroll
@@ -404,11 +437,19 @@ __global__ __launch_bounds__(64 * WM * WN * KG, KG > 2 ? KG : 2) void gemm_split
         if (worst != worst) bad = 1;
         __syncthreads();
         if (bad) {  // uniform
-            static_assert(KG * kGroupLds >= 2 * kBK * 4 * (BM + BN), "room for the fp32 tile");
-            auto Af = reinterpret_cast<float(*)[kBK * BM]>(lds);
-            auto Bf = reinterpret_cast<float(*)[kBK * BN]>(lds + 2 * kBK * BM * 4);
-            fp32_tile<TA, TB, BM, BN, WM, WN, EPI, 1, false, XF>(g, Ap, Bp, Cp, g.K, im, jn, Af, Bf);
-            return;
+            if (thread < 2) top[thread] = 0;
+            __syncthreads();
+            if (has_a) atomicMax(&top[0], __float_as_uint(SA::template largest<XF>(At, thread, g.lda, astep, g.K, xfa)));
+            if (has_b) atomicMax(&top[1], __float_as_uint(SB::template largest<XF>(Bt, thread, g.ldb, bstep, g.K, xfb)));
+            __syncthreads();
+            if (static_cast<double>(__uint_as_float(top[0])) * __uint_as_float(top[1]) * g.K >= 0x1p94 ||
+                !(__uint_as_float(top[0]) < 0x1p111f && __uint_as_float(top[1]) < 0x1p111f)) {
+                static_assert(KG * kGroupLds >= 2 * kBK * 4 * (BM + BN), "room for the fp32 tile");
+                auto Af = reinterpret_cast<float(*)[kBK * BM]>(lds);
+                auto Bf = reinterpret_cast<float(*)[kBK * BN]>(lds + 2 * kBK * BM * 4);
+                fp32_tile<TA, TB, BM, BN, WM, WN, EPI, 1, false, XF>(g, Ap, Bp, Cp, g.K, im, jn, Af, Bf);
+                return;
+            }
         }
     }
 
