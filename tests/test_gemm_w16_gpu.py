@@ -1,7 +1,9 @@
 """The 16x16x4 kernel (gemm_f32_w16: M and N multiples of 256, K of 32, at
 least one 256x256 tile per CU; the NN, NT and TN layouts, TT keeping the 32x32
 kernel): its corners against the f64 product, the column sums' fixed order and
-the separate epilogue kernels."""
+the separate epilogue kernels.  It has the products of fewer than 2.2e9
+operations and the NN ones whose B has 2^23 elements or more; the cases marked
+"bf16" run the same checks on the bf16 matrix cores (test_gemm_split_gpu.py)."""
 from __future__ import annotations
 
 import numpy as np
@@ -14,11 +16,13 @@ pytestmark = pytest.mark.gpu
 # (trans_a, trans_b, M, N, K, operand pitch pad, output pitch pad, C offset in floats)
 CASES = [
     (0, 0, 4096, 4096, 32, 0, 0, 0),     # one stage
-    (0, 0, 4096, 4096, 96, 0, 0, 0),     # an odd stage count
+    (0, 0, 4096, 4096, 96, 0, 0, 0),     # bf16
+    (0, 0, 256, 65536, 160, 0, 0, 0),    # an odd stage count
+    (0, 0, 256, 65536, 128, 4, 8, 1),
     (1, 0, 4096, 4096, 32, 0, 0, 0),
-    (1, 0, 4096, 4096, 160, 0, 0, 0),
+    (1, 0, 4096, 4096, 160, 0, 0, 0),    # bf16
     (0, 1, 4096, 4096, 32, 0, 0, 0),
-    (0, 1, 4096, 4096, 96, 0, 0, 0),
+    (0, 1, 4096, 4096, 96, 0, 0, 0),     # bf16
     (0, 0, 4096, 4096, 64, 4, 8, 0),     # operand and output pitches past the matrix
     (1, 0, 4096, 4096, 64, 12, 4, 0),
     (0, 1, 4096, 4096, 64, 8, 4, 0),
@@ -61,7 +65,7 @@ def test_w16_products(oracle, ta, tb, M, N, K, pad, cpad, coff):
         assert np.all(np.isnan(out[:, N:])), "the output pitch's padding was written"
 
 
-@pytest.mark.parametrize("K", [32, 96, 160])
+@pytest.mark.parametrize("K", [32, 64, 96, 160])  # (from 96 on bf16: column strips)
 def test_w16_column_sums(oracle, K):
     # the dW product with its bias gradient: chunks of 64 k rows across the
     # stages of 32, a last chunk of one stage when the stage count is odd

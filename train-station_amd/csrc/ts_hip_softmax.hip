@@ -393,7 +393,8 @@ static bool rows_are_long(size_t rows, size_t cols) {
 // More rows side by side while a row is short (their chains share the adds'
 // issue slots), then as many waves as the row needs at 8 columns a lane, the
 // rows of a workgroup halved and the columns of a lane doubled for the last.
-// From 2049 columns on the waves that wait for their turn show: where the rows
+// (The backward forms of 16 waves have 128 registers a lane for two operands
+// and spill 10, 8 and 20 of them.)  From 2049 columns on the waves that wait for their turn show: where the rows
 // fill the chip, half as many at 16 columns a lane (us forward / backward, 16384 x
 // 4000: 247 / 342 with eight, 199 / 210 with four; 2048 x 4000: 33 / 47 and 37 / 30;
 // 512 x 4000: 26 / 20 and 31 / 21).
