@@ -8,6 +8,9 @@
 // here the transpose is only a different index order in the global->LDS
 // staging, so no transposed copy ever exists.
 //
+// Most products of 2.2e9 operations and more run on the bf16 matrix cores
+// (ts_hip_gemm_split.h, chosen in split_plan); what follows has the others.
+//
 // Tiling.  A workgroup owns a BM x BN tile of C and walks K in steps of BK=16.
 // Its waves form a WM x WN grid; each wave owns (BM/WM) x (BN/WN) of C as a
 // grid of 32x32 v_mfma_f32_32x32x2_f32 accumulators.  Two shapes:
